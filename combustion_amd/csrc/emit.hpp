@@ -62,6 +62,8 @@ std::string emit_device_function(const ast::Linear& l, const std::vector<std::st
 extern const char* const rates_mixed_source;
 // FP64 rates kernel for large mechanisms (kernels/rates_tiled.hip).
 extern const char* const rates_tiled_source;
+// Rates kernel of teams of waves (kernels/rates_split.hip).
+extern const char* const rates_split_source;
 // Mixture-averaged transport kernel template (kernels/transport_tiled.hip).
 extern const char* const transport_tiled_source;
 // Surrogate network kernels (kernels/mlp.hip).

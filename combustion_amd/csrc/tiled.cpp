@@ -1,5 +1,6 @@
 // Mechanism-tiled forms, each launching its kernels on the caller's stream:
-//   fp64  (chemistry programs): the rates section as straight-line FP64 code, then transport_tiled in FP64;
+//   fp64  (chemistry programs): the rates section as straight-line FP64 code (one lane per state, or rates_split's
+//          teams of waves), then transport_tiled in FP64;
 //   mixed: rates_mixed (reaction tiles on BF16 MFMA, mechanism tables in device memory), then transport_tiled
 //          in FP32.
 // transport_tiled (kernels/transport_tiled.hip) evaluates the Wilke sums as three K×K MFMA contractions and the
@@ -15,6 +16,7 @@
 #include "emit.hpp"
 #include "forms.hpp"
 #include "mlp.hpp"
+#include "rates_split.hpp"
 #include "soa.hpp"
 
 namespace combustion {
@@ -515,34 +517,43 @@ void check_program(const ProgramView& p) {
 
 constexpr size_t kMaxStraightRatesSpecies = 64;
 
-// The rates section of a chemistry program as straight-line FP64 code (contraction and reciprocal division).
-std::string rates_straight_text(const ProgramView& p, bool fast) {
-  // Above 64 species the straight-line rates kernel spills kilobytes per lane to scratch (6.9 KB at K=160) and its
-  // code object runs to megabytes; the one run of the K=160 FP64 form on a GPU ended in a memory aperture violation
-  // during assembly whose cause was not established, so these mechanisms are refused here.
-  if (p.mechanism->species.len() > kMaxStraightRatesSpecies)
-    throw Unsupported("the straight-line FP64 rates kernel supports at most " + std::to_string(kMaxStraightRatesSpecies) +
-                      " species (this mechanism has " + std::to_string(p.mechanism->species.len()) + ")");
+// The rates section as one lane per state: straight-line FP64 code (contraction and reciprocal division).
+ast::Linear lean_rates(const ProgramView& p) {
   ChemistryOptions o;
   o.transport = false;
   o.lean_rates = true;
+  return ast::linearize(chemistry(*p.mechanism, nullptr, p.chemistry->scales, o));
+}
+
+// Kernel of the rates section up to 64 species, and for the team kernel its launch shape and tables.
+struct RatesText {
+  std::string name, source;
+  RatesSplit split;  // parts = 0: one lane per state
+};
+
+RatesText rates_text(const ProgramView& p, bool fast) {
+  // Above 64 species the straight-line sections grow to megabytes of code, and a straight-line K=160 kernel once ended
+  // in a memory aperture violation during assembly whose cause was not established, so these are refused here.
+  if (p.mechanism->species.len() > kMaxStraightRatesSpecies)
+    throw Unsupported("the straight-line FP64 rates kernel supports at most " + std::to_string(kMaxStraightRatesSpecies) +
+                      " species (this mechanism has " + std::to_string(p.mechanism->species.len()) + ")");
+  RatesText t;
+  t.name = fast ? "rates_fast" : "rates_fp64";
+  const ast::Linear l = lean_rates(p);
+  // A program of more live doubles than the 128 that two waves per SIMD hold goes to teams of waves (53 species: 0.80
+  // against 1.19 ms per 2^20 states at one wave per SIMD); a smaller one runs without their LDS traffic and barriers.
+  if (ast::peak_live(l) > 128) {
+    t.split = rates_split(*p.mechanism, t.name, fast);
+    t.source = t.split.source;
+    return t;
+  }
   StraightOptions so;
   so.reciprocal = true;
   so.newton_steps = 1;
   so.fast_transcendentals = fast;
   so.exp_poly = true;
-  const ast::Linear l = ast::linearize(chemistry(*p.mechanism, nullptr, p.chemistry->scales, o));
-  // A program that needs more than the 128 doubles of two waves per SIMD runs at one wave with its values in VGPRs,
-  // AGPRs and scratch; its clamped exp(-G_k/RT) values then live in LDS (K_a slots of 2 KB per block of 256). At
-  // K=53 (about 230 live doubles with the lean rates form) the kernel then needs no scratch and takes 1.25 ms per 2^20
-  // states against 1.30 ms with the values in registers; keeping some exp(+G_k/RT) values there too, a fence every
-  // 64 or 256 instructions, or two waves per SIMD with 40 slots (1.6 ms, 1.2 KB of scratch) were not faster, nor
-  // was reading the FP64 constants from a __constant__ table by scalar loads (3.2 k s_mov per wave fall to 1.8 k
-  // SALU instructions, but 1.48 ms against 1.18 ms: one wave per SIMD leaves the loads' latency exposed).
-  // Beyond 80 slots the values stay in registers.
-  if (ast::peak_live(l) > 128) so.lds_registers = gibbs_exponentials(l, true);
-  if (so.lds_registers.size() * so.block_size * 8 > 160 * 1024) so.lds_registers.clear();
-  return emit_straight(l, fast ? "rates_fast" : "rates_fp64", so);
+  t.source = emit_straight(l, t.name, so);
+  return t;
 }
 
 // rates_tiled with its tables in device memory; writes ω to out[0..Ka).
@@ -628,22 +639,36 @@ class RatesMixed {
   double *d_rcp_W_ = nullptr, *d_gibbs_ = nullptr, *d_split_ = nullptr;
 };
 
-// The rates section as straight-line FP64 code (with FP32 cores for exp and ln when fast); writes ω to out[0..Ka).
+// The rates section up to 64 species (with FP32 cores for exp and ln when fast); writes ω to out[0..Ka).
 class RatesStraight {
  public:
-  RatesStraight(const ProgramView& p, bool fast) {
-    const char* name = fast ? "rates_fast" : "rates_fp64";
-    kernel_.load(device::compile(rates_straight_text(p, fast), name, hip_options(true)), name);
+  RatesStraight(const ProgramView& p, bool fast) : t_(rates_text(p, fast)) {
+    kernel_.load(device::compile(t_.source, t_.name, hip_options(true)), t_.name);
+    if (t_.split.parts) {
+      d_rcp_W_ = upload(t_.split.rcp_W);
+      d_gibbs_ = upload(t_.split.gibbs);
+    }
+  }
+  ~RatesStraight() {
+    for (double* ptr : {d_rcp_W_, d_gibbs_})
+      if (ptr) (void)hipFree(ptr);
   }
   void launch(const double* const* in, double* const* out, size_t n, hipStream_t stream) {
-    unsigned n32 = (unsigned)n, offset = 0, block = 256;
-    void* args[] = {&in, &out, &n32, &offset};
-    unsigned grid = (unsigned)((n + block - 1) / block);
-    device::check(hipModuleLaunchKernel(kernel_.function, grid, 1, 1, block, 1, 1, 0, stream, args, nullptr), "launch rates_fp64");
+    unsigned n32 = (unsigned)n, offset = 0;
+    double pos = 6981463048192., neg = (double)cbrtf(3.40282347e38f);  // reaction.rs:244-256
+    void* straight[] = {&in, &out, &n32, &offset};
+    void* teams[] = {&in, &out, &n32, &d_rcp_W_, &d_gibbs_, &pos, &neg};
+    const unsigned block = t_.split.parts ? 64 * t_.split.teams * t_.split.parts : 256;
+    const unsigned states = t_.split.parts ? 64 * t_.split.teams : 256;
+    device::check(hipModuleLaunchKernel(kernel_.function, (unsigned)((n + states - 1) / states), 1, 1, block, 1, 1, 0, stream,
+                                        t_.split.parts ? teams : straight, nullptr),
+                  "launch rates");
   }
 
  private:
+  RatesText t_;
   device::Kernel kernel_;
+  double *d_rcp_W_ = nullptr, *d_gibbs_ = nullptr;
 };
 
 // Mechanisms up to 64 species take the transport section as straight-line code (one lane per state): at K=53 it
@@ -969,7 +994,7 @@ std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
   if (p.chemistry->options.rates)
     s += form == 2                      ? rates_mixed_text(mixed_tables(*p.mechanism))
          : tiled_rates(p, form_flags) ? rates_tiled_text(rates_tiled_tables(*p.mechanism))
-                                      : rates_straight_text(p, form == 3);
+                                      : rates_text(p, form == 3).source;
   if (p.chemistry->options.transport)
     s += "\n// ---- transport ----\n" + (straight_transport(p, form_flags) ? transport_straight_text(p, !mixed)
                                                          : transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed));
@@ -985,8 +1010,10 @@ void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
       device::compile(rates_mixed_text(mixed_tables(*p.mechanism)), "rates_mixed", hip_options(true));
     else if (tiled_rates(p, form_flags))
       device::compile(rates_tiled_text(rates_tiled_tables(*p.mechanism)), "rates_tiled", hip_options(true));
-    else
-      device::compile(rates_straight_text(p, form == 3), form == 3 ? "rates_fast" : "rates_fp64", hip_options(true));
+    else {
+      const RatesText t = rates_text(p, form == 3);
+      device::compile(t.source, t.name, hip_options(true));
+    }
   }
   if (p.chemistry->options.transport) {
     if (straight_transport(p, form_flags))
