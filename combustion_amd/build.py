@@ -12,12 +12,13 @@ CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libcombustion_amd.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 SOURCES = ["yaml.cpp", "mechanism.cpp", "ast.cpp", "reaction.cpp", "transport.cpp", "hip_emit.cpp", "device.cpp",
-           "forms.cpp", "rates_split.cpp", "tiled.cpp", "mlp.cpp", "export.cpp", "ignition.cpp", "host_jit.cpp", "jacobian.cpp", "integrator.cpp", "capi.cpp"]
+           "forms.cpp", "rates_split.cpp", "transport_split.cpp", "tiled.cpp", "mlp.cpp", "export.cpp", "ignition.cpp", "host_jit.cpp", "jacobian.cpp", "integrator.cpp", "capi.cpp"]
 
 
 KERNELS = {"rates_mixed_source": "rates_mixed.hip", "transport_tiled_source": "transport_tiled.hip",
            "mlp_source": "mlp.hip", "rosenbrock_source": "rosenbrock.hip", "rates_tiled_source": "rates_tiled.hip",
-           "surrogate_source": "surrogate.hip", "rates_split_source": "rates_split.hip"}
+           "surrogate_source": "surrogate.hip", "rates_split_source": "rates_split.hip",
+           "transport_split_source": "transport_split.hip"}
 
 
 def embed_kernels():

@@ -64,6 +64,8 @@ extern const char* const rates_mixed_source;
 extern const char* const rates_tiled_source;
 // Rates kernel of teams of waves (kernels/rates_split.hip).
 extern const char* const rates_split_source;
+// FP64 transport kernel of four waves per 64 states (kernels/transport_split.hip).
+extern const char* const transport_split_source;
 // Mixture-averaged transport kernel template (kernels/transport_tiled.hip).
 extern const char* const transport_tiled_source;
 // Surrogate network kernels (kernels/mlp.hip).

@@ -18,6 +18,7 @@
 #include "mlp.hpp"
 #include "rates_split.hpp"
 #include "soa.hpp"
+#include "transport_split.hpp"
 
 namespace combustion {
 
@@ -671,9 +672,9 @@ class RatesStraight {
   double *d_rcp_W_ = nullptr, *d_gibbs_ = nullptr;
 };
 
-// Mechanisms up to 64 species take the transport section as straight-line code (one lane per state): at K=53 it
-// issues fewer instructions per state than the tiled kernel, whose MFMA contractions do not pay for the
-// reciprocals and reductions around them. Larger mechanisms (a K² program) take transport_tiled.
+// Mechanisms up to 64 species take the transport section as straight-line code (one lane per state, or four waves per
+// 64 states): at K=53 it issues fewer instructions per state than the tiled kernel, whose MFMA contractions do not
+// pay for the reciprocals and reductions around them. Larger mechanisms (a K² program) take transport_tiled.
 // Mechanisms above kMaxStraightRatesSpecies (or any, with kFormTiledRates) take rates_tiled in forms 1 and 3.
 bool tiled_rates(const ProgramView& p, int form) {
   return p.mechanism->species.len() > kMaxStraightRatesSpecies || (form & kFormTiledRates);
@@ -682,7 +683,25 @@ bool tiled_rates(const ProgramView& p, int form) {
 // form | kFormTiledTransport sends every mechanism through transport_tiled (the MFMA contractions) instead.
 bool straight_transport(const ProgramView& p, int form) { return p.mechanism->species.len() <= 64 && !(form & kFormTiledTransport); }
 
-std::string transport_straight_text(const ProgramView& p, bool f64) {
+// Kernel of the transport section up to 64 species, with the tables of transport_split.
+struct TransportText {
+  std::string name, source;
+  TransportSplit split;  // empty tables: one lane per state
+};
+
+// Four waves per 64 states from this many species on (one lane per state below): at 2^19 states 0.15 against 0.17 ms
+// at 26 species, 0.218 either way at 32, 0.36 against 0.33 ms at 40. (On 4096 states, fewer than the lanes of the
+// chip, the four waves are ahead from 12 species on, by 1 us there and 33 us at 40.)
+constexpr size_t kSplitTransportSpecies = 32;
+
+TransportText transport_text(const ProgramView& p, bool f64) {
+  TransportText t;
+  t.name = f64 ? "transport_fp64" : "transport_f32";
+  if (f64 && p.mechanism->species.len() >= kSplitTransportSpecies) {
+    t.split = transport_split(*p.mechanism, polynomials(p));
+    t.source = t.split.source;
+    return t;
+  }
   ChemistryOptions o;
   o.rates = false;
   o.lean_transport = true;
@@ -691,28 +710,44 @@ std::string transport_straight_text(const ProgramView& p, bool f64) {
   so.reciprocal = f64;
   so.newton_steps = 1;
   so.f32 = !f64;
-  // FP64: the lean transport program fits two waves per SIMD (243 VGPRs, no AGPRs). FP32: three waves (168 VGPRs,
-  // one spilled register) beat two (246 VGPRs) by 1.5 % on the fast form's step at K=53.
+  // FP32: three waves per SIMD (168 VGPRs, one spilled register) beat two (246 VGPRs) by 1.5 % on the fast form's step
+  // at K=53.
   so.min_waves = f64 ? 2 : 3;
-  return emit_straight(ast::linearize(chemistry(*p.mechanism, p.chemistry->polynomials.get(), p.chemistry->scales, o)),
-                       f64 ? "transport_fp64" : "transport_f32", so);
+  t.source = emit_straight(ast::linearize(chemistry(*p.mechanism, p.chemistry->polynomials.get(), p.chemistry->scales, o)), t.name, so);
+  return t;
 }
 
 class TransportStraight {
  public:
-  TransportStraight(const ProgramView& p, bool f64) {
-    const char* name = f64 ? "transport_fp64" : "transport_f32";
-    kernel_.load(device::compile(transport_straight_text(p, f64), name, hip_options(true)), name);
+  TransportStraight(const ProgramView& p, bool f64) : t_(transport_text(p, f64)), rcp_T0_(1. / p.chemistry->scales.T0) {
+    kernel_.load(device::compile(t_.source, t_.name, hip_options(true)), t_.name);
+    if (split()) {
+      d_rcp_W_ = upload(t_.split.rcp_W);
+      d_W_ = upload(t_.split.W);
+      d_c_ = upload(t_.split.fit_c);
+      d_v_ = upload(t_.split.fit_v);
+    }
+  }
+  ~TransportStraight() {
+    for (double* ptr : {d_rcp_W_, d_W_, d_c_, d_v_})
+      if (ptr) (void)hipFree(ptr);
   }
   void launch(const double* const* in, double* const* out, size_t n, hipStream_t stream) {
-    unsigned n32 = (unsigned)n, offset = 0, block = 256;
-    void* args[] = {&in, &out, &n32, &offset};
-    unsigned grid = (unsigned)((n + block - 1) / block);
-    device::check(hipModuleLaunchKernel(kernel_.function, grid, 1, 1, block, 1, 1, 0, stream, args, nullptr), "launch transport");
+    unsigned n32 = (unsigned)n, offset = 0;
+    void* straight[] = {&in, &out, &n32, &offset};
+    void* teams[] = {&in, &out, &n32, &d_rcp_W_, &d_W_, &d_c_, &d_v_, &rcp_T0_};
+    const unsigned states = split() ? 64 : 256;
+    device::check(hipModuleLaunchKernel(kernel_.function, (unsigned)((n + states - 1) / states), 1, 1, 256, 1, 1, 0, stream,
+                                        split() ? teams : straight, nullptr),
+                  "launch transport");
   }
 
  private:
+  TransportText t_;
+  double rcp_T0_;
   device::Kernel kernel_;
+  double *d_rcp_W_ = nullptr, *d_W_ = nullptr, *d_c_ = nullptr, *d_v_ = nullptr;
+  bool split() const { return !t_.split.W.empty(); }
 };
 
 class Tiled : public SoAForm {
@@ -996,7 +1031,7 @@ std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
          : tiled_rates(p, form_flags) ? rates_tiled_text(rates_tiled_tables(*p.mechanism))
                                       : rates_text(p, form == 3).source;
   if (p.chemistry->options.transport)
-    s += "\n// ---- transport ----\n" + (straight_transport(p, form_flags) ? transport_straight_text(p, !mixed)
+    s += "\n// ---- transport ----\n" + (straight_transport(p, form_flags) ? transport_text(p, !mixed).source
                                                          : transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed));
   return s;
 }
@@ -1017,7 +1052,7 @@ void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
   }
   if (p.chemistry->options.transport) {
     if (straight_transport(p, form_flags))
-      device::compile(transport_straight_text(p, !mixed), mixed ? "transport_f32" : "transport_fp64", hip_options(true));
+      device::compile(transport_text(p, !mixed).source, mixed ? "transport_f32" : "transport_fp64", hip_options(true));
     else
       device::compile(transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed), "transport_tiled",
                       hip_options(true));
