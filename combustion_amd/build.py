@@ -6,10 +6,12 @@ time into the code-object cache by `precompile`). Usage: python -m combustion_am
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libcombustion_amd.so")
+TENSORS = os.path.join(HERE, "_tensors.so")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 SOURCES = ["yaml.cpp", "mechanism.cpp", "ast.cpp", "reaction.cpp", "transport.cpp", "hip_emit.cpp", "device.cpp",
            "forms.cpp", "rates_split.cpp", "transport_split.cpp", "tiled.cpp", "mlp.cpp", "export.cpp", "ignition.cpp", "host_jit.cpp", "jacobian.cpp", "integrator.cpp", "capi.cpp"]
@@ -40,6 +42,20 @@ def embed_kernels():
 HIP_SOURCES = ["noalloc.hip"]
 
 
+def build_tensors():
+    """Starts the compilation of the torch tensor helper (csrc/tensors.cpp) where torch is installed."""
+    try:
+        import torch
+        from torch.utils.cpp_extension import include_paths
+    except ImportError:
+        return None
+    libs = os.path.join(os.path.dirname(torch.__file__), "lib")
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}"]
+    cmd += ["-isystem" + d for d in include_paths() + [sysconfig.get_paths()["include"]]]
+    cmd += [os.path.join(CSRC, "tensors.cpp"), "-o", TENSORS + ".tmp", "-L" + libs, "-Wl,-rpath," + libs, "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    return "tensors.cpp", subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+
+
 def build(verbose=True):
     objs = []
     os.makedirs(os.path.join(HERE, "_build"), exist_ok=True)
@@ -57,6 +73,9 @@ def build(verbose=True):
                "-I" + os.path.join(ROCM, "include"), "-c", os.path.join(CSRC, src), "-o", obj]
         procs.append((src, subprocess.Popen(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)))
         objs.append(obj)
+    tensors = build_tensors()
+    if tensors:
+        procs.append(tensors)
     failed = False
     for src, p in procs:
         out, _ = p.communicate()
@@ -75,6 +94,8 @@ def build(verbose=True):
                                                   "-lamdhip64", "-lhiprtc", "-ldl"]
     subprocess.check_call(cmd)
     os.replace(tmp, LIB)
+    if tensors:
+        os.replace(TENSORS + ".tmp", TENSORS)
     return LIB
 
 

@@ -1,11 +1,14 @@
 // Launch plumbing shared by every form: SoA pointer tables in device memory, host-buffer staging, the ordering
 // of a module's calls across streams and kernel timing with HIP events on the caller's stream.
 #pragma once
+#include <cstring>
 #include <map>
+#include <memory>
 #include <vector>
 
 #include "device.hpp"
 #include "forms.hpp"
+#include "host_arrays.hpp"
 
 namespace combustion {
 
@@ -13,7 +16,9 @@ class SoAForm : public Form {
  public:
   SoAForm(int n_inputs, int n_outputs) : n_in_(n_inputs), n_out_(n_outputs) {}
   ~SoAForm() override {
-    for (auto& t : tables_) (void)hipFree(t.second);
+    for (void* slab : slabs_) (void)hipFree(slab);
+    if (staging_) (void)hipHostFree(staging_);
+    if (copy_) (void)hipStreamDestroy(copy_);
     if (start_) (void)hipEventDestroy(start_);
     if (stop_) (void)hipEventDestroy(stop_);
     if (done_) (void)hipEventDestroy(done_);
@@ -27,6 +32,18 @@ class SoAForm : public Form {
       return;
     }
     if (!on_device) {
+      // A form with work memory of its own reports on whole calls (the surrogate's fallback count), so its states go in
+      // one slice; the others in slices that stay within the staging.
+      if (!host_) host_ = std::make_unique<HostArrays>(n_in_, n_out_);
+      if (work_bytes(n) == 0 && host_->sliceable(inputs, n, outputs)) {
+        if (kernel_ms) *kernel_ms = 0;
+        host_->call(inputs, n, outputs, [&](const double* const* din, size_t count, double* const* dout, hipStream_t slot) {
+          float ms = 0;
+          run(din, count, dout, slot, kernel_ms ? &ms : nullptr);
+          if (kernel_ms) *kernel_ms += ms;
+        });
+        return;
+      }
       std::vector<double*> din(n_in_, nullptr), dout(n_out_, nullptr);
       struct Free {
         std::vector<double*>& a;
@@ -64,15 +81,11 @@ class SoAForm : public Form {
   // module keeps between its kernels (the surrogate's fallback list) is never shared by two calls in flight. Not
   // while the stream is being captured into a graph: the caller orders captured work.
   void order_after_previous_call(hipStream_t stream) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    device::check(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing");
-    if (capture != hipStreamCaptureStatusNone) return;
+    if (capturing(stream)) return;
     if (done_ && stream != last_stream_) device::check(hipStreamWaitEvent(stream, done_, 0), "hipStreamWaitEvent");
   }
   void mark_call_done(hipStream_t stream) {
-    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
-    device::check(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing");
-    if (capture != hipStreamCaptureStatusNone) return;
+    if (capturing(stream)) return;
     if (!done_) device::check(hipEventCreateWithFlags(&done_, hipEventDisableTiming), "hipEventCreateWithFlags");
     device::check(hipEventRecord(done_, stream), "hipEventRecord");
     last_stream_ = stream;
@@ -80,30 +93,54 @@ class SoAForm : public Form {
 
  private:
   // One device table of the arrays' pointers per distinct set of arrays, written once when the set is first seen and
-  // never rewritten while the module lives: a launch still in flight on any stream, or a graph captured from this
+  // not rewritten until its set is forgotten: a launch still in flight on any stream, or a graph captured from this
   // module, keeps reading the table it was given. Past kMaxTables sets the device is synchronized and the tables
-  // are freed (graphs captured before that point must then be captured again).
+  // are used again (graphs captured before that point must then be captured again).
   static constexpr size_t kMaxTables = 1024;
   int n_in_, n_out_;
   std::map<std::vector<const void*>, void*> tables_;
   hipEvent_t start_ = nullptr, stop_ = nullptr, done_ = nullptr;
   hipStream_t last_stream_ = nullptr;
+  std::unique_ptr<HostArrays> host_;
+
+  // The null stream is never captured, and asking costs a runtime call.
+  static bool capturing(hipStream_t stream) {
+    if (!stream) return false;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    device::check(hipStreamIsCapturing(stream, &capture), "hipStreamIsCapturing");
+    return capture != hipStreamCaptureStatusNone;
+  }
+
+  // Tables come from slabs of kSlabTables (at most kMaxTables in all), their contents through pinned memory on a stream
+  // of the module's own: a first call on new arrays pays neither an allocation nor a wait for the work before it.
+  static constexpr size_t kSlabTables = 64;
+  std::vector<void*> slabs_, free_tables_;
+  void* staging_ = nullptr;
+  hipStream_t copy_ = nullptr;
 
   void* table_for(const std::vector<const void*>& ptrs) {
     auto it = tables_.find(ptrs);
     if (it != tables_.end()) return it->second;
-    if (tables_.size() >= kMaxTables) {
-      device::check(hipDeviceSynchronize(), "hipDeviceSynchronize");
-      for (auto& t : tables_) device::check(hipFree(t.second), "hipFree table");
-      tables_.clear();
+    const size_t bytes = (ptrs.size() * sizeof(void*) + 255) / 256 * 256;
+    if (free_tables_.empty()) {
+      if (tables_.size() >= kMaxTables) {
+        device::check(hipDeviceSynchronize(), "hipDeviceSynchronize");
+        for (auto& t : tables_) free_tables_.push_back(t.second);
+        tables_.clear();
+      } else {
+        void* slab = nullptr;
+        device::check(hipMalloc(&slab, kSlabTables * bytes), "hipMalloc tables");
+        slabs_.push_back(slab);
+        for (size_t i = kSlabTables; i-- > 0;) free_tables_.push_back((char*)slab + i * bytes);
+      }
     }
-    void* table = nullptr;
-    device::check(hipMalloc(&table, ptrs.size() * sizeof(void*)), "hipMalloc table");
-    const hipError_t e = hipMemcpy(table, ptrs.data(), ptrs.size() * sizeof(void*), hipMemcpyHostToDevice);
-    if (e != hipSuccess) {
-      (void)hipFree(table);
-      device::check(e, "hipMemcpy table");
-    }
+    if (!copy_) device::check(hipStreamCreateWithFlags(&copy_, hipStreamNonBlocking), "hipStreamCreateWithFlags");
+    if (!staging_) device::check(hipHostMalloc(&staging_, bytes, hipHostMallocDefault), "hipHostMalloc");
+    void* table = free_tables_.back();
+    std::memcpy(staging_, ptrs.data(), ptrs.size() * sizeof(void*));
+    device::check(hipMemcpyAsync(table, staging_, ptrs.size() * sizeof(void*), hipMemcpyHostToDevice, copy_), "hipMemcpyAsync table");
+    device::check(hipStreamSynchronize(copy_), "hipStreamSynchronize table");
+    free_tables_.pop_back();
     tables_.emplace(ptrs, table);
     return table;
   }
@@ -115,11 +152,11 @@ class SoAForm : public Form {
     return ptrs;
   }
 
-  // Frees the table of a pointer set whose launches have completed.
+  // Gives back the table of a pointer set whose launches have completed.
   void forget_table(const double* const* inputs, double* const* outputs) {
     auto it = tables_.find(pointer_set(inputs, outputs));
     if (it == tables_.end()) return;
-    device::check(hipFree(it->second), "hipFree table");
+    free_tables_.push_back(it->second);
     tables_.erase(it);
   }
 

@@ -376,6 +376,22 @@ def _pointer(x):
     raise TypeError("inputs must be numpy arrays or torch device tensors")
 
 
+_addresses = None
+
+
+def _tensor_addresses():
+    """The native helper that reads a list of tensors' addresses (csrc/tensors.cpp); loaded once torch tensors are used."""
+    global _addresses
+    if _addresses is None:
+        try:
+            import torch  # noqa: F401 (the helper links against it)
+            from ._tensors import addresses
+        except ImportError as e:
+            raise ImportError(f"the tensor helper is missing: build it with `python -m combustion_amd.build` ({e})") from e
+        _addresses = addresses
+    return _addresses
+
+
 class Module:
     """The callable device::assemble returns (device.rs:59): module(inputs) -> outputs (SoA)."""
 
@@ -395,25 +411,32 @@ class Module:
         if len(inputs) != self.program.n_inputs:
             raise ValueError(f"expected {self.program.n_inputs} inputs, got {len(inputs)}")
         n = len(inputs[0])
-        ptrs = [_pointer(x) for x in inputs]
-        on_device = ptrs[0][1]
-        if any(d != on_device for _, d in ptrs):
-            raise ValueError("inputs must all be on the host or all on the device")
-        if any(len(x) != n for x in inputs):
-            raise ValueError("all inputs must have the same length")
+        n_in, n_out = self.program.n_inputs, self.program.n_outputs
+        in_arr, out_arr = (C.c_void_p * n_in)(), (C.c_void_p * n_out)()
+        # contiguous float64 CUDA tensors are read in one native pass, anything else (host arrays, and what is refused)
+        # one by one
+        on_device = getattr(inputs[0], "is_cuda", False) and _tensor_addresses()(inputs, C.addressof(in_arr), n) == n
+        if not on_device:
+            ptrs = [_pointer(x) for x in inputs]
+            on_device = ptrs[0][1]
+            if any(d != on_device for _, d in ptrs):
+                raise ValueError("inputs must all be on the host or all on the device")
+            if any(len(x) != n for x in inputs):
+                raise ValueError("all inputs must have the same length")
+            in_arr[:] = [p for p, _ in ptrs]
         if outputs is None:
             if on_device:
                 import torch
-                outputs = [torch.empty(n, dtype=torch.float64, device=inputs[0].device) for _ in range(self.program.n_outputs)]
+                outputs = [torch.empty(n, dtype=torch.float64, device=inputs[0].device) for _ in range(n_out)]
             else:
-                outputs = [np.empty(n) for _ in range(self.program.n_outputs)]
-        optrs = [_pointer(x) for x in outputs]
-        if any(d != on_device for _, d in optrs) or len(outputs) != self.program.n_outputs:
-            raise ValueError("outputs must match the inputs' placement and the program's output count")
-        in_arr = (C.c_void_p * len(ptrs))(*[p for p, _ in ptrs])
-        out_arr = (C.c_void_p * len(optrs))(*[p for p, _ in optrs])
+                outputs = [np.empty(n) for _ in range(n_out)]
+        if len(outputs) != n_out or not on_device or _tensor_addresses()(outputs, C.addressof(out_arr), n) != n:
+            optrs = [_pointer(x) for x in outputs]
+            if any(d != on_device for _, d in optrs) or len(outputs) != n_out:
+                raise ValueError("outputs must match the inputs' placement and the program's output count")
+            out_arr[:] = [p for p, _ in optrs]
         ms = C.c_float(0)
-        _check(lib().cb_hip_call(self._h, in_arr, len(ptrs), n, out_arr, len(optrs), int(on_device), stream,
+        _check(lib().cb_hip_call(self._h, in_arr, n_in, n, out_arr, n_out, int(on_device), stream,
                                  C.byref(ms) if time_kernel else None))
         if time_kernel:
             self.last_kernel_ms = ms.value
