@@ -3,10 +3,12 @@
 #pragma once
 #include <hip/hip_runtime_api.h>
 
+#include <algorithm>
 #include <condition_variable>
 #include <cstring>
 #include <functional>
 #include <mutex>
+#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -75,8 +77,9 @@ class CopyTeam {
   }
 };
 
-// Staging of one module: two slots of pinned and device memory with a stream each, allocated with the first call on
-// host arrays, grown to at most kSlotBytes each and given back with the module.
+// Staging of one module: two slots of pinned and device memory, allocated with the first call on host arrays, grown to
+// at most kSlotBytes each (or one group of 64 states) and given back with the module. The slots' streams live as long
+// as a call: streams share the GPU's few hardware queues, and an idle one may sit in the way of another module's.
 class HostArrays {
  public:
   static constexpr size_t kSlotBytes = size_t(16) << 20;
@@ -104,13 +107,23 @@ class HostArrays {
     const size_t most = std::max<size_t>(64, kSlotBytes / (rows * sizeof(double)) / 64 * 64);
     const size_t slices = (n + most - 1) / most, per = ((n + slices - 1) / slices + 63) / 64 * 64;
     reserve(per);
-    CopyTeam team(n * rows * sizeof(double) < kThreadedBytes ? 0 : helpers());
-    struct Drain {  // nothing is in flight on return, an exception's included
+    struct Streams {
       HostArrays& h;
-      ~Drain() {
-        for (Slot& s : h.slots_) (void)hipStreamSynchronize(s.stream);
+      void create() {
+        for (Slot& s : h.slots_) device::check(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking), "hipStreamCreateWithFlags");
       }
-    } drain{*this};
+      ~Streams() {  // nothing is in flight on return, an exception's included
+        for (Slot& s : h.slots_) {
+          if (!s.stream) continue;
+          (void)hipStreamSynchronize(s.stream);
+          (void)hipStreamDestroy(s.stream);
+          s.stream = nullptr;
+        }
+      }
+    };
+    Streams streams{*this};
+    streams.create();
+    CopyTeam team(n * rows * sizeof(double) < kThreadedBytes ? 0 : helpers());
     auto finish = [&](size_t slice) {
       Slot& s = slots_[slice % 2];
       const size_t first = slice * per, count = std::min(per, n - first);
@@ -151,7 +164,6 @@ class HostArrays {
     release();
     const size_t bytes = (size_t)(n_in_ + n_out_) * states * sizeof(double);
     for (Slot& s : slots_) {
-      device::check(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking), "hipStreamCreateWithFlags");
       device::check(hipHostMalloc((void**)&s.pinned, bytes, hipHostMallocDefault), "hipHostMalloc");
       device::check(hipMalloc((void**)&s.device, bytes), "hipMalloc staging");
     }
@@ -159,7 +171,6 @@ class HostArrays {
   }
   void release() {
     for (Slot& s : slots_) {
-      if (s.stream) (void)hipStreamDestroy(s.stream);
       if (s.pinned) (void)hipHostFree(s.pinned);
       if (s.device) (void)hipFree(s.device);
       s = Slot{};

@@ -17,8 +17,6 @@ class SoAForm : public Form {
   SoAForm(int n_inputs, int n_outputs) : n_in_(n_inputs), n_out_(n_outputs) {}
   ~SoAForm() override {
     for (void* slab : slabs_) (void)hipFree(slab);
-    if (staging_) (void)hipHostFree(staging_);
-    if (copy_) (void)hipStreamDestroy(copy_);
     if (start_) (void)hipEventDestroy(start_);
     if (stop_) (void)hipEventDestroy(stop_);
     if (done_) (void)hipEventDestroy(done_);
@@ -111,12 +109,12 @@ class SoAForm : public Form {
     return capture != hipStreamCaptureStatusNone;
   }
 
-  // Tables come from slabs of kSlabTables (at most kMaxTables in all), their contents through pinned memory on a stream
-  // of the module's own: a first call on new arrays pays neither an allocation nor a wait for the work before it.
+  // Tables come from slabs of kSlabTables (at most kMaxTables in all): a first call on new arrays pays one copy and, at a
+  // slab's first table only, an allocation. The copy is complete before the launch, so that any stream or graph may
+  // read the table; it is not on a stream of its own, because the few hardware queues would then be shared by the
+  // streams that the kernels run on.
   static constexpr size_t kSlabTables = 64;
   std::vector<void*> slabs_, free_tables_;
-  void* staging_ = nullptr;
-  hipStream_t copy_ = nullptr;
 
   void* table_for(const std::vector<const void*>& ptrs) {
     auto it = tables_.find(ptrs);
@@ -134,12 +132,8 @@ class SoAForm : public Form {
         for (size_t i = kSlabTables; i-- > 0;) free_tables_.push_back((char*)slab + i * bytes);
       }
     }
-    if (!copy_) device::check(hipStreamCreateWithFlags(&copy_, hipStreamNonBlocking), "hipStreamCreateWithFlags");
-    if (!staging_) device::check(hipHostMalloc(&staging_, bytes, hipHostMallocDefault), "hipHostMalloc");
     void* table = free_tables_.back();
-    std::memcpy(staging_, ptrs.data(), ptrs.size() * sizeof(void*));
-    device::check(hipMemcpyAsync(table, staging_, ptrs.size() * sizeof(void*), hipMemcpyHostToDevice, copy_), "hipMemcpyAsync table");
-    device::check(hipStreamSynchronize(copy_), "hipStreamSynchronize table");
+    device::check(hipMemcpy(table, ptrs.data(), ptrs.size() * sizeof(void*), hipMemcpyHostToDevice), "hipMemcpy table");
     free_tables_.pop_back();
     tables_.emplace(ptrs, table);
     return table;

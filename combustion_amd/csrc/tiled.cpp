@@ -758,6 +758,7 @@ class Tiled : public SoAForm {
     const auto& o = p.chemistry->options;
     const int form = form_flags & kFormBase;
     const bool f64 = form == 1;
+    species_ = p.mechanism->species.len();
     if (o.rates) {
       n_rates_ = (int)p.mechanism->active;
       if (form == 2)
@@ -782,12 +783,20 @@ class Tiled : public SoAForm {
   }
 
  protected:
-  // The rates and transport kernels read the same inputs and write disjoint outputs: the transport kernel runs on a
-  // second stream of the module's (default priority), forked from and joined back into the caller's stream, so that
-  // the two kernels' blocks share the CUs at the ends of each launch (2.27 against 2.32 ms per 2^20 states at K=53).
+  // The rates and transport kernels read the same inputs and write disjoint outputs. Where both take long, the
+  // transport kernel runs on a second stream of the module's (default priority), forked from and joined back into the
+  // caller's stream, so that the two kernels' blocks share the CUs (1.74 against 1.76 ms per 2^20 states at K=53; 4096
+  // states of 160 species in the mixed form, whose few blocks leave most of the chip idle, 0.37 against 0.53 ms). The
+  // fork and join take about 25 us on the GPU and 15 us of the host's time, so that kernels of that length run one
+  // after the other instead: up to kForkWork (48 k states of 53 species, where they take 45 us each; 4096 states of 10
+  // species, 8 us each, take 15 instead of 41 us), except for the large-mechanism and MFMA rates kernels, whose
+  // smallest batches already take 50 us from 32 species on.
+  static constexpr size_t kForkWork = size_t(1) << 27, kForkSpecies = 32;
   void launch(const double* const* in, double* const* out, size_t n, const Launch& how) override {
     hipStream_t stream = how.stream;
-    const bool both = (mixed_ || fp64_ || tiled_rates_) && (straight_ || transport_) && !how.single_stream;
+    const bool slow = (mixed_ || tiled_rates_) && species_ >= kForkSpecies;
+    const bool both = (mixed_ || fp64_ || tiled_rates_) && (straight_ || transport_) && !how.single_stream &&
+                      (slow || n >= kForkWork / (species_ * species_));
     hipStream_t ts = stream;
     if (both) {
       if (!side_) {
@@ -818,6 +827,7 @@ class Tiled : public SoAForm {
   std::unique_ptr<TransportStraight> straight_;
   std::unique_ptr<TransportTiled> transport_;
   int n_rates_ = 0;
+  size_t species_ = 0;
   hipStream_t side_ = nullptr;
   hipEvent_t fork_ = nullptr, join_ = nullptr;
 };
