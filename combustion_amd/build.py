@@ -20,7 +20,8 @@ SOURCES = ["yaml.cpp", "mechanism.cpp", "ast.cpp", "reaction.cpp", "transport.cp
 KERNELS = {"rates_mixed_source": "rates_mixed.hip", "transport_tiled_source": "transport_tiled.hip",
            "mlp_source": "mlp.hip", "rosenbrock_source": "rosenbrock.hip", "rates_tiled_source": "rates_tiled.hip",
            "surrogate_source": "surrogate.hip", "rates_split_source": "rates_split.hip",
-           "transport_split_source": "transport_split.hip"}
+           "transport_split_source": "transport_split.hip",
+           "transport_pairs_source": "transport_pairs.hip"}
 
 
 def embed_kernels():

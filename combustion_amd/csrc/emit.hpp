@@ -66,6 +66,8 @@ extern const char* const rates_tiled_source;
 extern const char* const rates_split_source;
 // FP64 transport kernel of four waves per 64 states (kernels/transport_split.hip).
 extern const char* const transport_split_source;
+// FP64 transport kernel of sixteen waves per 64 states (kernels/transport_pairs.hip).
+extern const char* const transport_pairs_source;
 // Mixture-averaged transport kernel template (kernels/transport_tiled.hip).
 extern const char* const transport_tiled_source;
 // Surrogate network kernels (kernels/mlp.hip).

@@ -4,7 +4,8 @@
 //   mixed: rates_mixed (reaction tiles on BF16 MFMA, mechanism tables in device memory), then transport_tiled
 //          in FP32.
 // transport_tiled (kernels/transport_tiled.hip) evaluates the Wilke sums as three K×K MFMA contractions and the
-// binary-diffusion polynomials as (pairs × D)·(D × states) MFMA tiles.
+// binary-diffusion polynomials as (pairs × D)·(D × states) MFMA tiles; in FP64 it gives way to transport_split (32 to 64
+// species) and transport_pairs (65 to 160).
 #include <algorithm>
 #include <array>
 #include <cstdlib>
@@ -750,6 +751,40 @@ class TransportStraight {
   bool split() const { return !t_.split.W.empty(); }
 };
 
+// transport_pairs with its tables in device memory; writes [λ, μ, D_0..D_{K-1}] to out[0..K+2).
+class TransportPairsKernel {
+ public:
+  TransportPairsKernel(TransportPairs t, double T0) : t_(std::move(t)), rcp_T0_(1. / T0) {
+    kernel_.load(device::compile(t_.source, "transport_tiled", hip_options(true)), "transport_tiled");
+    for (const auto* v : {&t_.rcp_W, &t_.W, &t_.fit_c, &t_.fit_v, &t_.columns, &t_.rows, &t_.pairs}) tables_.push_back(upload(*v));
+    d_offset_ = upload(t_.offset);
+  }
+  ~TransportPairsKernel() {
+    for (double* ptr : tables_) (void)hipFree(ptr);
+    if (d_offset_) (void)hipFree(d_offset_);
+  }
+  void launch(const double* const* in, double* const* out, size_t n, hipStream_t stream) {
+    unsigned n32 = (unsigned)n;
+    void* args[] = {&in, &out, &n32, &tables_[0], &tables_[1], &tables_[2], &tables_[3], &tables_[4], &tables_[5], &tables_[6], &d_offset_, &rcp_T0_};
+    device::check(hipModuleLaunchKernel(kernel_.function, (unsigned)((n + 63) / 64), 1, 1, 64 * t_.waves, 1, 1, 0, stream, args, nullptr),
+                  "launch transport");
+  }
+
+ private:
+  TransportPairs t_;
+  double rcp_T0_;
+  device::Kernel kernel_;
+  std::vector<double*> tables_;
+  unsigned* d_offset_ = nullptr;
+};
+
+// Mechanisms above 64 species take transport_pairs in FP64 where its LDS holds them (up to 160 species: 0.99 against 2.09 ms
+// per 2^17 states there), transport_tiled beyond, in FP32 and on lists of states.
+TransportPairs pairs_of(const ProgramView& p, int form_flags) {
+  if ((form_flags & kFormBase) != 1 || (form_flags & kFormTiledTransport) || p.mechanism->species.len() <= 64) return {};
+  return transport_pairs(*p.mechanism, polynomials(p));
+}
+
 class Tiled : public SoAForm {
  public:
   // form 1: FP64 rates and transport; 2: MFMA mixed rates, FP32 transport; 3: FP32-core rates, FP32 transport.
@@ -769,7 +804,10 @@ class Tiled : public SoAForm {
         fp64_ = std::make_unique<RatesStraight>(p, form == 3);
     }
     if (o.transport) {
-      if (straight_transport(p, form_flags))
+      TransportPairs pairs = pairs_of(p, form_flags);
+      if (!pairs.source.empty())
+        pairs_ = std::make_unique<TransportPairsKernel>(std::move(pairs), p.chemistry->scales.T0);
+      else if (straight_transport(p, form_flags))
         straight_ = std::make_unique<TransportStraight>(p, f64);
       else
         transport_ = std::make_unique<TransportTiled>(p, f64);
@@ -795,7 +833,7 @@ class Tiled : public SoAForm {
   void launch(const double* const* in, double* const* out, size_t n, const Launch& how) override {
     hipStream_t stream = how.stream;
     const bool slow = (mixed_ || tiled_rates_) && species_ >= kForkSpecies;
-    const bool both = (mixed_ || fp64_ || tiled_rates_) && (straight_ || transport_) && !how.single_stream &&
+    const bool both = (mixed_ || fp64_ || tiled_rates_) && (straight_ || transport_ || pairs_) && !how.single_stream &&
                       (slow || n >= kForkWork / (species_ * species_));
     hipStream_t ts = stream;
     if (both) {
@@ -814,6 +852,7 @@ class Tiled : public SoAForm {
     if (tiled_rates_) tiled_rates_->launch(in, out, n, stream);
     if (straight_) straight_->launch(in, out + n_rates_, n, ts);
     if (transport_) transport_->launch(in, out + n_rates_, n, ts);
+    if (pairs_) pairs_->launch(in, out + n_rates_, n, ts);
     if (both) {
       device::check(hipEventRecord(join_, side_), "hipEventRecord");
       device::check(hipStreamWaitEvent(stream, join_, 0), "hipStreamWaitEvent");
@@ -826,6 +865,7 @@ class Tiled : public SoAForm {
   std::unique_ptr<RatesTiled> tiled_rates_;
   std::unique_ptr<TransportStraight> straight_;
   std::unique_ptr<TransportTiled> transport_;
+  std::unique_ptr<TransportPairsKernel> pairs_;
   int n_rates_ = 0;
   size_t species_ = 0;
   hipStream_t side_ = nullptr;
@@ -1040,9 +1080,13 @@ std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
     s += form == 2                      ? rates_mixed_text(mixed_tables(*p.mechanism))
          : tiled_rates(p, form_flags) ? rates_tiled_text(rates_tiled_tables(*p.mechanism))
                                       : rates_text(p, form == 3).source;
-  if (p.chemistry->options.transport)
-    s += "\n// ---- transport ----\n" + (straight_transport(p, form_flags) ? transport_text(p, !mixed).source
-                                                         : transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed));
+  if (p.chemistry->options.transport) {
+    s += "\n// ---- transport ----\n";
+    const TransportPairs pairs = pairs_of(p, form_flags);
+    if (!pairs.source.empty()) s += pairs.source;
+    else if (straight_transport(p, form_flags)) s += transport_text(p, !mixed).source;
+    else s += transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed);
+  }
   return s;
 }
 
@@ -1061,7 +1105,10 @@ void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
     }
   }
   if (p.chemistry->options.transport) {
-    if (straight_transport(p, form_flags))
+    const TransportPairs pairs = pairs_of(p, form_flags);
+    if (!pairs.source.empty())
+      device::compile(pairs.source, "transport_tiled", hip_options(true));
+    else if (straight_transport(p, form_flags))
       device::compile(transport_text(p, !mixed).source, mixed ? "transport_f32" : "transport_fp64", hip_options(true));
     else
       device::compile(transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed), "transport_tiled",

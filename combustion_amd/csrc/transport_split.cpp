@@ -237,4 +237,56 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
   return t;
 }
 
+TransportPairs transport_pairs(const Mechanism& m, const Polynomials& p) {
+  TransportPairs t;
+  const std::vector<double>& W = m.species.molar_mass;
+  const size_t K = W.size(), D = p.D, waves = t.waves, slots = (K + waves - 1) / waves, half = slots / 2;
+  const std::vector<double> G = wilke_factor(W);
+  const size_t R = G.size() / K, KC = (K + 7) / 8 * 8;
+  // the two LDS arrays, the rows of the waves' partial sums in them, and fits that can be normalised
+  bool fits = slots >= 4 && (2 * K - 1) * 64 * sizeof(double) <= 160 * 1024 && K > 3 * waves && 3 * R <= K && D >= 2;
+  for (size_t k = 0; k < K && fits; k++)
+    for (size_t j = 0; j < k; j++) fits = fits && p.diffusivityITVT[(k * K + j) * D] != 0.;
+  if (!fits) return t;
+  std::ostringstream head;
+  head << "#define K " << K << "\n#define KA " << m.active << "\n#define R " << R << "\n#define DD " << D << "\n#define WAVES " << waves << "\n";
+  t.source = head.str() + transport_pairs_source;
+  for (size_t k = 0; k < K; k++) {
+    t.rcp_W.push_back(1. / W[k]);
+    t.W.push_back(W[k]);
+    for (size_t d = 0; d < D; d++) {
+      t.fit_c.push_back(p.conductivityIVT[k * D + d]);
+      t.fit_v.push_back(p.VviscosityIVVT[k * D + d] / std::sqrt(std::sqrt(W[k])));
+    }
+  }
+  t.columns.assign(R * KC, 0.);
+  for (size_t r = 0; r < R; r++)
+    for (size_t j = 0; j < K; j++) t.columns[r * KC + j] = G[j * R + r] * std::sqrt(W[j] / 8.);
+  t.rows.assign(waves * R * slots, 0.);
+  for (size_t w = 0; w < waves; w++)
+    for (size_t r = 0; r < R; r++)
+      for (size_t i = 0; w + waves * i < K; i++) t.rows[(w * R + r) * slots + i] = G[(w + waves * i) * R + r] / std::sqrt(W[w + waves * i]);
+  // pairs of the wave's slot i (species k) with species j, a slot without species giving no term
+  auto pair = [&](size_t k, size_t j) {
+    const double* c = k < K && j < K ? &p.diffusivityITVT[(k * K + j) * D] : nullptr;
+    for (size_t d = 1; d < D; d++) t.pairs.push_back(c ? c[d] / c[0] : 0.);
+    t.pairs.push_back(c ? 1. / c[0] : 0.);
+  };
+  for (size_t w = 0; w < waves; w++) {
+    t.offset.push_back((unsigned)t.pairs.size());
+    auto column = [&](size_t j, size_t n) {
+      for (size_t i = 0; i < n; i++) pair(w + waves * i, j);
+    };
+    for (size_t a = 1; a < slots; a++)
+      for (size_t b = 0; b < a; b++) pair(w + waves * a, w + waves * b);
+    for (size_t phase = 1; phase < waves / 2; phase++)
+      for (size_t j = (w + phase) % waves; j < K; j += waves) column(j, slots);
+    if (w < waves / 2)
+      for (size_t j = w + waves / 2; j < K; j += waves) column(j, half);
+    else
+      for (size_t j = w - waves / 2 + waves * half; j < K; j += waves) column(j, slots);
+  }
+  return t;
+}
+
 }  // namespace combustion
