@@ -1,7 +1,9 @@
 // Multilayer perceptron of the transport surrogate: parameter layout, workspace and the launch sequences of the
 // forward pass, the backward pass of a mean-squared-error loss and Adam (kernels/mlp.hip). The network is
 // in -> width (SiLU) -> ... -> width (SiLU) -> out, with `depth` hidden layers; feature dimensions are padded to
-// multiples of 64 (padding columns of inputs, targets and weights are zero and stay zero).
+// multiples of 64 (padding columns of inputs, targets and weights are zero and stay zero). Up to 576 features a layer the
+// forward pass is one launch and the backward pass three for every two layers (their data gradients, their weight
+// gradients over ranges of states, the sum of the ranges); wider networks run layer by layer.
 #include "mlp.hpp"
 
 #include <algorithm>
@@ -13,6 +15,7 @@ namespace combustion {
 
 namespace {
 constexpr long kChunk = 1024;  // states per weight-gradient partial sum
+constexpr unsigned kRows = 64;  // states per block of the fused kernels
 long pad64(long x) { return (x + 63) / 64 * 64; }
 unsigned blocks(long n, unsigned per) { return (unsigned)((n + per - 1) / per); }
 }  // namespace
@@ -39,6 +42,7 @@ Mlp::Mlp(int n_in, int width, int depth, int n_out) : n_in_(n_in), n_out_(n_out)
   in_pad_ = lay.in_pad;
   out_pad_ = lay.out_pad;
   n_params_ = lay.n_params;
+  widest_ = std::max({in_pad_, (long)width_, out_pad_});
   for (const auto& L : lay.layers) layers_.push_back({L.in, L.out, L.w, L.b});
   image_ = device::compile(mlp_source, "mlp", hip_options(true));  // kept while the module is loaded
   device::check(hipModuleLoadData(&module_, image_.data()), "hipModuleLoadData mlp");
@@ -49,6 +53,9 @@ Mlp::Mlp(int n_in, int width, int depth, int n_out) : n_in_(n_in), n_out_(n_out)
   get(to_bf16_, "mlp_to_bf16");
   get(mse_, "mlp_mse_grad");
   get(adam_, "mlp_adam");
+  get(forward_, "mlp_forward");
+  get(backward_, "mlp_backward");
+  get(weights_, "mlp_weights");
 }
 
 Mlp::~Mlp() {
@@ -102,6 +109,14 @@ void Mlp::gemm(int mode, long M, long N, long Kd, const uint16_t* A, long sam, l
 void Mlp::forward(const float* params, const uint16_t* params16, const float* x, long n, float* y, void* ws, hipStream_t s) const {
   if (n <= 0) return;
   Views v = views(ws, n);
+  if (fused()) {
+    int in = (int)in_pad_, width = width_, out = (int)out_pad_, depth = depth_, ld = (int)widest_ + 16;
+    long layer_bytes = depth_ > 1 ? (char*)v.z[1] - (char*)v.z[0] : 0;  // z and h of a layer follow each other, layer by layer
+    void* a[] = {&x, &params, &params16, &n, &in, &width, &out, &depth, &ld, &v.h[0], &v.z[0], &v.h[1], &layer_bytes, &y};
+    device::check(hipModuleLaunchKernel(forward_, blocks(n, kRows), 1, 1, 512, 1, 1, fused_lds(), s, a, nullptr),
+                  "launch mlp_forward");
+    return;
+  }
   long total = n * in_pad_;
   void* a0[] = {&x, &total, &v.h[0]};
   device::check(hipModuleLaunchKernel(to_bf16_, blocks(total, 256), 1, 1, 256, 1, 1, 0, s, a0, nullptr), "launch mlp_to_bf16");
@@ -113,9 +128,54 @@ void Mlp::forward(const float* params, const uint16_t* params16, const float* x,
   }
 }
 
+// Two layers at a time from the output, the room that the workspace has for gradients by pre-activations (n × widest
+// twice): the upper one's in g[0], the lower one's in g[1], where the next pair's launch finds it. The ranges of states of
+// the weight gradients are as many as the workspace's partial sums hold for two layers, of at least 256 states each, and
+// one range writes its sums in place. (2^14 states of the 55-256-256-256-55 network: 12 ranges, 240 blocks a launch.)
+void Mlp::backward_fused(const uint16_t* params16, const float* y, const float* target, long n, const Views& v, float* grad,
+                         hipStream_t s) const {
+  struct LayerGradient {
+    const uint16_t *g, *h;
+    int rows, cols;
+    long w, b;
+  };
+  int out = (int)out_pad_, valid = n_out_, width = width_, ld = (int)widest_ + 16;
+  uint16_t *ghi = v.g[0], *glo = v.g[1];
+  const float* none = nullptr;
+  for (int hi = depth_; hi >= 0; hi -= 2) {
+    const bool pair = hi > 0;
+    int from_loss = hi == depth_;
+    const uint16_t *wabove = from_loss ? nullptr : params16 + layers_[hi + 1].w, *whi = params16 + layers_[hi].w;
+    const float *zhi = from_loss ? none : v.z[hi], *zlo = pair ? v.z[hi - 1] : none;
+    void* a0[] = {&y, &target, &n, &out, &valid, &from_loss, &width, &wabove, &whi, &zhi, &zlo, &ghi, &glo, &ld};
+    device::check(hipModuleLaunchKernel(backward_, blocks(n, kRows), 1, 1, 512, 1, 1, fused_lds(), s, a0, nullptr),
+                  "launch mlp_backward");
+    const long base = layers_[pair ? hi - 1 : hi].w, top = layers_[hi].b + layers_[hi].out;
+    auto layer = [&](int l, const uint16_t* g) {
+      const Layer& L = layers_[l];
+      return LayerGradient{g, v.h[l], (int)L.out, (int)L.in, L.w - base, L.b - base};
+    };
+    LayerGradient upper = layer(hi, ghi), lower = pair ? layer(hi - 1, glo) : upper;
+    long tiles = (long)(upper.rows / 64) * (upper.cols / 64) + (pair ? (long)(lower.rows / 64) * (lower.cols / 64) : 0);
+    long size = top - base, room = (long)blocks(n, kChunk) * max_layer_params() / size;
+    int parts = (int)std::max(1L, std::min<long>(room, blocks(n, 256)));
+    long range = ((n + parts - 1) / parts + 63) / 64 * 64;
+    parts = (int)((n + range - 1) / range);
+    float *partial = v.partial, *to = parts == 1 ? grad + base : partial;
+    void* a1[] = {&upper, &lower, &n, &parts, &range, &to, &size};
+    device::check(hipModuleLaunchKernel(weights_, (unsigned)(tiles * parts), 1, 1, 1024, 1, 1, 0, s, a1, nullptr), "launch mlp_weights");
+    if (parts > 1) {
+      float* gw = grad + base;
+      void* a2[] = {&partial, &size, &parts, &gw};
+      device::check(hipModuleLaunchKernel(reduce_, blocks(size, 256), 1, 1, 256, 1, 1, 0, s, a2, nullptr), "launch mlp_reduce");
+    }
+  }
+}
+
 void Mlp::backward_mse(const uint16_t* params16, const float* y, const float* target, long n, void* ws, float* grad, hipStream_t s) const {
   if (n <= 0) return;
   Views v = views(ws, n);
+  if (fused()) return backward_fused(params16, y, target, n, v, grad, s);
   long total = n * out_pad_, ld = out_pad_, valid = n_out_;
   void* a0[] = {&y, &target, &n, &ld, &valid, &v.g[0]};
   device::check(hipModuleLaunchKernel(mse_, blocks(total, 256), 1, 1, 256, 1, 1, 0, s, a0, nullptr), "launch mlp_mse_grad");

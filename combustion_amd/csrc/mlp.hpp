@@ -57,12 +57,20 @@ class Mlp {
   void gemm(int mode, long M, long N, long Kd, const uint16_t* A, long sam, long sak, const uint16_t* B, long sbn, long sbk, const float* bias,
             const float* zprev, float* zout, uint16_t* hout, long ldc, float* partial, unsigned parts, hipStream_t s) const;
 
+  // forward and backward in fused kernels (see mlp.cpp), or layer by layer
+  bool fused() const { return widest_ <= kFusedWidth; }
+  void backward_fused(const uint16_t* params16, const float* y, const float* target, long n, const Views& v, float* grad, hipStream_t s) const;
+
+  // two tiles of 64 states in 160 KB of LDS
+  unsigned fused_lds() const { return (unsigned)(2 * 64 * (widest_ + 16)) * 2; }
+  static constexpr long kFusedWidth = 576;
   int n_in_, n_out_, width_, depth_;
+  long widest_;
   long in_pad_, out_pad_, n_params_;
   std::vector<Layer> layers_;
   hipModule_t module_ = nullptr;
   std::vector<char> image_;
-  hipFunction_t gemm_, reduce_, colsum_, to_bf16_, mse_, adam_;
+  hipFunction_t gemm_, reduce_, colsum_, to_bf16_, mse_, adam_, forward_, backward_, weights_;
 };
 
 }  // namespace combustion
