@@ -46,6 +46,9 @@ struct StraightOptions {
   // Output o of state id is stored at out[o][id · output_stride] (with out[o] = base + o and the stride the number of
   // outputs, state by state).
   unsigned output_stride = 1;
+  // A device function of one state instead of a kernel: void name(const double* in, double* out), the inputs and outputs
+  // consecutive (no groups, no LDS registers); with helpers false, without the functions that the first of several emits.
+  bool device_function = false, helpers = true;
 };
 // Straight-line kernel: signature (const double* const* in, double* const* out, unsigned n, unsigned offset).
 std::string emit_straight(const ast::Linear& l, const std::string& name, const StraightOptions& o);

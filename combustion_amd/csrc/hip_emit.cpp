@@ -21,7 +21,7 @@ std::string literal(double x) {
 std::string emit_straight(const ast::Linear& l, const std::string& name, const StraightOptions& o) {
   using ast::LOp;
   std::ostringstream s;
-  if (o.reciprocal && !o.f32) {
+  if (o.helpers && o.reciprocal && !o.f32) {
     s << "__device__ __forceinline__ double rcp64(double b) {\n"
          "  double r = __builtin_amdgcn_rcp(b);\n";
     for (unsigned i = 0; i < o.newton_steps; i++)
@@ -30,7 +30,7 @@ std::string emit_straight(const ast::Linear& l, const std::string& name, const S
     s << "  return r;\n"
          "}\n";
   }
-  if (o.fast_transcendentals && !o.f32)
+  if (o.helpers && o.fast_transcendentals && !o.f32)
     s << "__device__ __forceinline__ double exp_wide(double x) {\n"
          "  const double y = x * 1.4426950408889634;\n"
          "  const double n = __builtin_fmin(__builtin_fmax(__builtin_rint(y), -1100.0), 1100.0);\n"
@@ -42,7 +42,7 @@ std::string emit_straight(const ast::Linear& l, const std::string& name, const S
          "  const double m = __longlong_as_double((b & 0x000FFFFFFFFFFFFFLL) | 0x3FF0000000000000LL);\n"
          "  return ((double)e + (double)__builtin_amdgcn_logf((float)m)) * 0.6931471805599453;\n"
          "}\n";
-  if (o.exp_poly && !o.f32 && !o.fast_transcendentals)
+  if (o.helpers && o.exp_poly && !o.f32 && !o.fast_transcendentals)
     s << "__device__ __forceinline__ double exp64(double x) {\n"
          "  x = __builtin_fmin(__builtin_fmax(x, -746.0), 710.0);\n"
          "  const double t = __builtin_fma(x, 0x1.71547652b82fep+0, 0x1.8p+52);\n"
@@ -67,13 +67,19 @@ std::string emit_straight(const ast::Linear& l, const std::string& name, const S
     s << "__device__ __forceinline__ float rcp32(float b) { return __builtin_amdgcn_rcpf(b); }\n"
          "__device__ __forceinline__ float exp32(float x) { return __builtin_amdgcn_exp2f(x * 1.4426950408889634f); }\n"
          "__device__ __forceinline__ float log32(float x) { return __builtin_amdgcn_logf(x) * 0.6931471805599453f; }\n";
-  s << "extern \"C\" __global__ void __launch_bounds__(" << o.block_size;
-  if (o.min_waves) s << ", " << o.min_waves;
-  s << ") ";
-  s << name
-    << "(const double* const* __restrict__ in, double* const* __restrict__ out, unsigned n, unsigned offset) {\n"
-    << "  const unsigned id = offset + blockIdx.x * blockDim.x + threadIdx.x;\n";
   const bool grouped = o.group_table >= 0;
+  if (o.device_function) {
+    if (grouped || o.f32 || !o.lds_registers.empty() || o.output_stride != 1)
+      throw ast::Error("emit: a device function has one state's inputs and outputs in FP64");
+    s << "__device__ __forceinline__ void " << name << "(const double* __restrict__ in, double* __restrict__ out) {\n";
+  } else {
+    s << "extern \"C\" __global__ void __launch_bounds__(" << o.block_size;
+    if (o.min_waves) s << ", " << o.min_waves;
+    s << ") ";
+    s << name
+      << "(const double* const* __restrict__ in, double* const* __restrict__ out, unsigned n, unsigned offset) {\n"
+      << "  const unsigned id = offset + blockIdx.x * blockDim.x + threadIdx.x;\n";
+  }
   auto option = [&](const std::vector<int32_t>& v, int32_t r) { return r < (int32_t)v.size() ? v[r] : -1; };
   if (grouped && (o.group_size == 0 || o.block_size % o.group_size != 0 || o.group_stride == 0))
     throw ast::Error("emit: the group size must divide the block size, and groups need values");
@@ -85,7 +91,7 @@ std::string emit_straight(const ast::Linear& l, const std::string& name, const S
         (option(o.increment_offset, r) >= 0 &&
          (option(o.group_offset, r) < 0 || option(o.increment_state, r) < 0 || option(o.increment_state, r) >= (int32_t)o.group_size)))
       throw ast::Error("emit: a group offset past the group's values, without a group, or an increment for no member");
-  if (!grouped) s << "  if (id >= n) return;\n";
+  if (!grouped && !o.device_function) s << "  if (id >= n) return;\n";
   // LDS-resident registers: slot of each, -1 for the others.
   std::vector<int32_t> slot(l.n_registers, -1);
   int32_t n_slots = 0;
@@ -125,9 +131,10 @@ std::string emit_straight(const ast::Linear& l, const std::string& name, const S
     for (int32_t r = 0; r < l.n_input; r++) increments |= option(o.increment_offset, r) >= 0;
     if (increments) s << "  const unsigned member = id % " << o.group_size << "u;\n";
   }
-  const std::string out_index = o.output_stride == 1 ? "[id]" : "[(size_t)id * " + std::to_string(o.output_stride) + "u]";
+  const std::string index = o.device_function ? "" : "[id]";
+  const std::string out_index = o.output_stride == 1 ? index : "[(size_t)id * " + std::to_string(o.output_stride) + "u]";
   for (int i = 0; i < l.n_input; i++)
-    if (option(o.group_offset, i) < 0) s << "  const " << F << " r" << i << " = (" << F << ")in[" << i << "][id];\n";
+    if (option(o.group_offset, i) < 0) s << "  const " << F << " r" << i << " = (" << F << ")in[" << i << "]" << index << ";\n";
   std::vector<char> loaded(l.n_input, 0);
   auto load_grouped = [&](int32_t r) {  // a grouped input, loaded before its first use
     if (r >= l.n_input || option(o.group_offset, r) < 0 || loaded[r]) return;

@@ -20,6 +20,10 @@ extern const char* const rosenbrock_source;
 
 namespace {
 constexpr int kPollEvery = 8;
+// Waves of rosenbrock_steps up to which it is faster than the separate kernels: its programs use one lane in seven, so
+// that beyond four waves a SIMD the chip is busy with them (six species, us a step, whole against separate: 1000 reactors
+// 29 against 86, 10^4 38 against 87, 2·10^4 57 against 88, 5·10^4 101 against 99, 2·10^5 349 against 260).
+constexpr size_t kWholeStepsWaves = 4096;
 
 // One wave per block for the right-hand-side and Jacobian programs: a launch over n reactors then spreads over
 // every CU (2^14 reactors in blocks of 256 states would occupy 64 of the 256 CUs).
@@ -93,7 +97,7 @@ struct IntegratorPrograms {
   bool differences;
   ast::Function rhs_function, jacobian_function, shared_function, varying_function;
   ast::Linear rhs_linear, jacobian_linear, shared_linear, varying_linear;
-  std::string step_source;
+  std::string step_source, whole_source;  // whole_source: empty unless a system's steps may run in one kernel
   IntegratorPrograms(const Mechanism& mech, int flags) : m((int)mech.species.len() + 1) {
     if (m > 64) throw Unsupported("the batched integrator holds a reactor's state in one wave: at most 63 species");
     const int jac = flags & kJacobianMask;
@@ -122,6 +126,15 @@ struct IntegratorPrograms {
     if (differences) src << "#define JAC_DIFFERENCES 1\n#define COPIES " << copies_per_reactor(m) << "\n";
     src << rosenbrock_source;
     step_source = src.str();
+    // whole steps in one kernel: RODAS4 with the Jacobian program, for the sizes whose Jacobian fits the registers
+    if (!differences && m <= kAnalyticMaxState && !(flags & (kOneSystemPerWave | kMethodOde23s))) {
+      StraightOptions o = straight_options(1, kProgramBlock);
+      o.device_function = true;
+      whole_source = emit_straight(jacobian_linear, "reactor_jacobian", o);
+      o.helpers = false;
+      whole_source += emit_straight(rhs_linear, "reactor_rhs", o);
+      whole_source += "#define WHOLE_STEPS 1\n" + step_source;
+    }
   }
 };
 
@@ -135,6 +148,7 @@ void compile_integrator(std::shared_ptr<const Mechanism> m, int flags) {
                      varying_options(p.varying_linear, p.m));
   }
   device::compile(p.step_source, "rosenbrock", hip_options(true));
+  if (!p.whole_source.empty()) device::compile(p.whole_source, "rosenbrock_steps", hip_options(true));
 }
 
 Integrator::Integrator(std::shared_ptr<const Mechanism> m, double rtol, double atol_T, double atol_Y, int flags)
@@ -165,10 +179,13 @@ Integrator::Integrator(std::shared_ptr<const Mechanism> m, double rtol, double a
                                  varying_options(varying_linear_, m_));
   }
   step_.load(device::compile(p.step_source, "rosenbrock", hip_options(true)), "rosenbrock");
+  whole_ = !p.whole_source.empty();
+  if (whole_) whole_steps_.load(device::compile(p.whole_source, "rosenbrock_steps", hip_options(true)), "rosenbrock_steps");
 }
 
 Integrator::~Integrator() {
   release();
+  if (whole_running_) (void)hipFree(whole_running_);
   if (fork_) (void)hipEventDestroy(fork_);
   if (join_) (void)hipEventDestroy(join_);
   for (hipEvent_t e : polled_)
@@ -187,17 +204,24 @@ void Integrator::release() {
   last_status_ = nullptr;
 }
 
+// What the polls of either path need: the events and the pinned words behind which the running counts arrive.
+void Integrator::prepare_polls() {
+  if (host_count_) return;
+  for (hipEvent_t& e : polled_)
+    if (!e) device::check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreateWithFlags");
+  device::check(hipHostMalloc((void**)&host_count_, 2 * sizeof(unsigned), hipHostMallocDefault), "hipHostMalloc");
+}
+
 void Integrator::prepare(double* y, const double* P, const int* status, size_t n) {
   if (n == n_ && y == last_y_ && P == last_P_ && status == last_status_) return;
   device::check(hipDeviceSynchronize(), "hipDeviceSynchronize");
   release();
+  prepare_polls();
   if (sides_.empty()) {
     sides_.resize(parts_count_ - 1);
     for (hipStream_t& s : sides_) device::check(hipStreamCreateWithFlags(&s, hipStreamNonBlocking), "hipStreamCreateWithFlags");
     device::check(hipEventCreateWithFlags(&fork_, hipEventDisableTiming), "hipEventCreateWithFlags");
     device::check(hipEventCreateWithFlags(&join_, hipEventDisableTiming), "hipEventCreateWithFlags");
-    for (hipEvent_t& e : polled_) device::check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreateWithFlags");
-    device::check(hipHostMalloc((void**)&host_count_, 2 * sizeof(unsigned), hipHostMallocDefault), "hipHostMalloc");
   }
   const size_t m = (size_t)m_;
   auto alloc = [&](size_t bytes) {
@@ -284,10 +308,65 @@ void Integrator::join_sides(hipStream_t stream) {
   }
 }
 
+// Counts the systems still running after `taken` steps: the count waits for every part's steps so far; it goes to pinned
+// memory behind an event, and the host reads the previous poll's count instead, which the GPU has usually passed: the GPU
+// never idles for the round trip. Reactors that are not running are left alone, so the steps launched after a poll that
+// found none running change nothing, and the call reports the steps up to that poll (in `found`, returning true).
+bool Integrator::poll(unsigned* running, const int* status, unsigned n, long taken, hipStream_t stream, hipFunction_t clear,
+                      hipFunction_t count_running, bool sides, int& polls, long (&polled_steps)[2], long& found) {
+  const int slot = polls & 1;
+  if (sides) join_sides(stream);
+  unsigned* count = running + slot;
+  void* cargs[] = {&count};
+  device::check(hipModuleLaunchKernel(clear, 1, 1, 1, 64, 1, 1, 0, stream, cargs, nullptr), "launch rosenbrock_clear");
+  void* rargs[] = {&n, &status, &count};
+  device::check(hipModuleLaunchKernel(count_running, (n + 255) / 256, 1, 1, 256, 1, 1, 0, stream, rargs, nullptr), "launch rosenbrock_running");
+  if (sides) {
+    // the other parts go on after the count only, so that it sees every part at this step, not later ones
+    device::check(hipEventRecord(fork_, stream), "hipEventRecord");
+    for (hipStream_t s : sides_) device::check(hipStreamWaitEvent(s, fork_, 0), "hipStreamWaitEvent");
+  }
+  device::check(hipMemcpyAsync(host_count_ + slot, count, sizeof(unsigned), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
+  device::check(hipEventRecord(polled_[slot], stream), "hipEventRecord");
+  polled_steps[slot] = taken;
+  if (++polls < 2) return false;
+  device::check(hipEventSynchronize(polled_[slot ^ 1]), "hipEventSynchronize");
+  if (host_count_[slot ^ 1] != 0) return false;
+  found = polled_steps[slot ^ 1];
+  return true;
+}
+
+// kPollEvery steps a launch, on the caller's stream.
+long Integrator::advance_whole(double* y, const double* P, double* t, double* h, int* status, unsigned* steps, size_t n, double t_end,
+                               int max_steps, hipStream_t stream) {
+  prepare_polls();
+  if (!whole_running_) device::check(hipMalloc((void**)&whole_running_, 256), "hipMalloc integrator");
+  hipFunction_t running = nullptr, clear = nullptr;
+  device::check(hipModuleGetFunction(&running, whole_steps_.module, "rosenbrock_running"), "hipModuleGetFunction");
+  device::check(hipModuleGetFunction(&clear, whole_steps_.module, "rosenbrock_clear"), "hipModuleGetFunction");
+  unsigned n32 = (unsigned)n;
+  size_t ld = n;
+  double te = t_end, rtol = rtol_, atol0 = atol_T_, atol = atol_Y_;
+  long taken = 0, polled_steps[2] = {0, 0};
+  int polls = 0;
+  while (taken < max_steps) {
+    int count = (int)std::min<long>(kPollEvery, max_steps - taken);
+    void* args[] = {&count, &n32, &ld, &P, &y, &t, &h, &status, &steps, &te, &rtol, &atol0, &atol};
+    device::check(hipModuleLaunchKernel(whole_steps_.function, (n32 + systems_per_wave_ - 1) / systems_per_wave_, 1, 1, 64, 1, 1, 0, stream,
+                                        args, nullptr),
+                  "launch rosenbrock_steps");
+    taken += count;
+    if (poll(whole_running_, status, n32, taken, stream, clear, running, false, polls, polled_steps, taken)) break;
+  }
+  device::check(hipStreamSynchronize(stream), "hipStreamSynchronize");
+  return taken;
+}
+
 long Integrator::advance(double* y, const double* P, double* t, double* h, int* status, unsigned* steps, size_t n, double t_end,
                          int max_steps, hipStream_t stream) {
   if (n == 0) return 0;
   if (n >= (size_t(1) << 31)) throw ArgumentError("at most 2^31 - 1 reactors");
+  if (whole_ && n <= kWholeStepsWaves * systems_per_wave_) return advance_whole(y, P, t, h, status, steps, n, t_end, max_steps, stream);
   prepare(y, P, status, n);
   hipFunction_t running = nullptr, clear = nullptr, copies_kernel = nullptr, stage = nullptr;
   device::check(hipModuleGetFunction(&stage, step_.module, "rosenbrock_stage"), "hipModuleGetFunction");
@@ -340,30 +419,7 @@ long Integrator::advance(double* y, const double* P, double* t, double* h, int* 
     }
     taken++;
     if ((step + 1) % kPollEvery == 0 || step + 1 == max_steps) {
-      // the count waits for every part's steps so far; it goes to pinned memory behind an event, and the host reads
-      // the previous poll's count instead, which the GPU has usually passed: the GPU never idles for the round trip.
-      // Reactors that are not running are left alone, so the steps launched after a poll that found none running
-      // change nothing, and the call reports the steps up to that poll.
-      const int slot = polls & 1;
-      join_sides(stream);
-      unsigned* count = running_ + slot;
-      void* cargs[] = {&count};
-      device::check(hipModuleLaunchKernel(clear, 1, 1, 1, 64, 1, 1, 0, stream, cargs, nullptr), "launch rosenbrock_clear");
-      void* rargs[] = {&n32, &status, &count};
-      device::check(hipModuleLaunchKernel(running, (n32 + 255) / 256, 1, 1, 256, 1, 1, 0, stream, rargs, nullptr), "launch rosenbrock_running");
-      // the other parts go on after the count only, so that it sees every part at this step, not later ones
-      device::check(hipEventRecord(fork_, stream), "hipEventRecord");
-      for (hipStream_t s : sides_) device::check(hipStreamWaitEvent(s, fork_, 0), "hipStreamWaitEvent");
-      device::check(hipMemcpyAsync(host_count_ + slot, count, sizeof(unsigned), hipMemcpyDeviceToHost, stream), "hipMemcpyAsync");
-      device::check(hipEventRecord(polled_[slot], stream), "hipEventRecord");
-      polled_steps[slot] = taken;
-      if (++polls >= 2) {
-        device::check(hipEventSynchronize(polled_[slot ^ 1]), "hipEventSynchronize");
-        if (host_count_[slot ^ 1] == 0) {
-          taken = polled_steps[slot ^ 1];
-          break;
-        }
-      }
+      if (poll(running_, status, n32, taken, stream, clear, running, true, polls, polled_steps, taken)) break;
     }
   }
   // every step launched is complete on return

@@ -74,12 +74,20 @@ class Integrator {
   hipEvent_t fork_ = nullptr, join_ = nullptr;
   hipEvent_t polled_[2] = {nullptr, nullptr};  // the last two polls' counts copied to host_count_ (pinned)
   unsigned* host_count_ = nullptr;
+  bool whole_ = false;  // whole steps in one kernel (rosenbrock_steps)
+  device::Kernel whole_steps_;
+  unsigned* whole_running_ = nullptr;  // its running counts
   const double* last_y_ = nullptr;
   const double* last_P_ = nullptr;
   const int* last_status_ = nullptr;
   void release();
   void prepare(double* y, const double* P, const int* status, size_t n);
+  void prepare_polls();
   void join_sides(hipStream_t stream);
+  bool poll(unsigned* running, const int* status, unsigned n, long taken, hipStream_t stream, hipFunction_t clear, hipFunction_t count_running,
+            bool sides, int& polls, long (&polled_steps)[2], long& found);
+  long advance_whole(double* y, const double* P, double* t, double* h, int* status, unsigned* steps, size_t n, double t_end, int max_steps,
+                     hipStream_t stream);
 };
 
 }  // namespace combustion

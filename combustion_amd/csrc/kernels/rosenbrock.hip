@@ -99,6 +99,61 @@ __device__ __forceinline__ double solve(const double (&a)[M], int pos, const int
   return x;
 }
 
+// Factors W (lane i holds row i in a) in place with partial pivoting: perm[k] the row chosen at step k (the same in every
+// lane of a system), pos the step at which row i was chosen (-1 before); returns row i's pivot.
+__device__ __forceinline__ double factor(double (&a)[M], int (&perm)[M], int& pos, bool row, int i, int base) {
+  double diag = 1.0;  // this row's pivot, U_i[pos]
+#pragma unroll
+  for (int k = 0; k < M; k++) {
+    // pivot: the largest |a[k]| over the rows not yet chosen (ties to the lowest row)
+    const double key = row && pos < 0 ? fabs(a[k]) : -1.0;
+#if P == 1
+    // the high words of |a| (plus one; 0 for rows already chosen) order the rows as |a| does up to ties, which
+    // the rare case resolves over the tied lanes in ascending order
+    const unsigned hi = row && pos < 0 ? (unsigned)(__builtin_bit_cast(unsigned long long, key) >> 32) + 1u : 0u;
+    unsigned long long tied = __builtin_amdgcn_ballot_w64(hi == wave_max(hi));
+    int p = (int)__builtin_ctzll(tied);
+    if (tied & (tied - 1)) {
+      double best = -1.0;
+      while (tied) {
+        const int l = (int)__builtin_ctzll(tied);
+        tied &= tied - 1;
+        const double v = lane_value(key, l);
+        if (v > best) {
+          best = v;
+          p = l;
+        }
+      }
+    }
+#else
+    double best = -2.0;
+    int p = 0;
+#pragma unroll
+    for (int r = 0; r < M; r++) {
+      const double kr = __shfl(key, base + r);
+      if (kr > best) {
+        best = kr;
+        p = r;
+      }
+    }
+#endif
+    perm[k] = p;
+    if (row && i == p) pos = k;
+    // the pivot row's entries are read from its lane by every lane (outside the branch: the pivot row is final)
+    const double pivot = row_value(a[k], p, base);
+    if (row && i == p) diag = pivot;
+    const bool eliminate = row && pos < 0;
+    const double l = eliminate ? a[k] / pivot : 0.0;
+    if (eliminate) a[k] = l;
+#pragma unroll
+    for (int j = k + 1; j < M; j++) {
+      const double pj = row_value(a[j], p, base);
+      a[j] = __builtin_fma(-l, pj, a[j]);  // l = 0 leaves the rows already chosen as they are (finite pj)
+    }
+  }
+  return diag;
+}
+
 // Difference quotients (the dense Jacobian of the reference's CVODE path, cvode/lib.rs:17-47): component j of a
 // system's state is increased by inc_j = √ε max(|y_j|, atol_j / rtol).
 __device__ __forceinline__ double increment(double yj, int j, double rtol, double atol0, double atol) {
@@ -164,6 +219,24 @@ __device__ __forceinline__ double rodas_stage(const double (&a)[M], int pos, con
 #define FACTOR_MAX 5.0
 #endif
 
+// The scaled error of a step to y1 with the error estimate err, over the lane's system.
+__device__ __forceinline__ double error_ratio(double err, double y0, double y1, bool row, int i, int base, double rtol, double atol0,
+                                              double atol) {
+  // step control: accept when the scaled error's root mean square over the components is at most 1 (the weighted
+  // RMS norm of CVODE); the next h from it
+  const double scale = (i == 0 ? atol0 : atol) + rtol * fmax(fabs(y0), fabs(y1));
+  double q = row ? err / scale : 0.0;
+  q *= q;
+  if (!(q == q)) q = 1e300;  // a NaN (a singular W, say) rejects the step
+  return sqrt(system_sum(q, base) * (1.0 / M));
+}
+
+// The step after one of hs.
+__device__ __forceinline__ double next_step(double hs, double ratio, bool accept) {
+  const double by = fmin(FACTOR_MAX, fmax(0.2, 0.9 * pow(fmax(ratio, 1e-12), -1.0 / ERROR_ORDER)));
+  return hs * (accept ? by : fmin(by, 0.5));
+}
+
 // Phase 1 (FIRST) or a later phase (phase >= 2): two kernels, so that the later phases, which hold no LU in
 // progress, are compiled to their own (smaller) register count.
 template <bool FIRST>
@@ -228,55 +301,10 @@ __device__ __forceinline__ void rosenbrock_phase(int phase, unsigned n, size_t l
 #endif
       a[j] = (row ? -hs * GAMMA * Jij : 0.0) + (row && i == j ? 1.0 : 0.0);
     }
-    double diag = 1.0;  // this row's pivot, U_i[pos]
+    const double diag = factor(a, perm, pos, row, i, base);
+    if (active && i == 0) {
 #pragma unroll
-    for (int k = 0; k < M; k++) {
-      // pivot: the largest |a[k]| over the rows not yet chosen (ties to the lowest row)
-      const double key = row && pos < 0 ? fabs(a[k]) : -1.0;
-#if P == 1
-      // the high words of |a| (plus one; 0 for rows already chosen) order the rows as |a| does up to ties, which
-      // the rare case resolves over the tied lanes in ascending order
-      const unsigned hi = row && pos < 0 ? (unsigned)(__builtin_bit_cast(unsigned long long, key) >> 32) + 1u : 0u;
-      unsigned long long tied = __builtin_amdgcn_ballot_w64(hi == wave_max(hi));
-      int p = (int)__builtin_ctzll(tied);
-      if (tied & (tied - 1)) {
-        double best = -1.0;
-        while (tied) {
-          const int l = (int)__builtin_ctzll(tied);
-          tied &= tied - 1;
-          const double v = lane_value(key, l);
-          if (v > best) {
-            best = v;
-            p = l;
-          }
-        }
-      }
-#else
-      double best = -2.0;
-      int p = 0;
-#pragma unroll
-      for (int r = 0; r < M; r++) {
-        const double kr = __shfl(key, base + r);
-        if (kr > best) {
-          best = kr;
-          p = r;
-        }
-      }
-#endif
-      perm[k] = p;
-      if (active && i == 0) perm_s[k] = p;
-      if (row && i == p) pos = k;
-      // the pivot row's entries are read from its lane by every lane (outside the branch: the pivot row is final)
-      const double pivot = row_value(a[k], p, base);
-      if (row && i == p) diag = pivot;
-      const bool eliminate = row && pos < 0;
-      const double l = eliminate ? a[k] / pivot : 0.0;
-      if (eliminate) a[k] = l;
-#pragma unroll
-      for (int j = k + 1; j < M; j++) {
-        const double pj = row_value(a[j], p, base);
-        a[j] = __builtin_fma(-l, pj, a[j]);  // l = 0 leaves the rows already chosen as they are (finite pj)
-      }
+      for (int k = 0; k < M; k++) perm_s[k] = perm[k];
     }
     const double rd = 1.0 / diag;
     if (active) {
@@ -348,23 +376,16 @@ __device__ __forceinline__ void rosenbrock_phase(int phase, unsigned n, size_t l
   const double y0 = row ? y[(size_t)ir * ld + sv] : 0.0, y1 = row ? ys[(size_t)ir * ld + sv] : 0.0;
   const double err = hs * (x1 - 2.0 * x2 + x3) * (1.0 / 6.0);
 #endif
-  // step control: accept when the scaled error's root mean square over the components is at most 1 (the weighted
-  // RMS norm of CVODE); the next h from it
-  const double scale = (i == 0 ? atol0 : atol) + rtol * fmax(fabs(y0), fabs(y1));
-  double q = row ? err / scale : 0.0;
-  q *= q;
-  if (!(q == q)) q = 1e300;  // a NaN (a singular W, say) rejects the step
-  const double ratio = sqrt(system_sum(q, base) * (1.0 / M));
+  const double ratio = error_ratio(err, y0, y1, row, i, base, rtol, atol0, atol);
   if (!active) return;
   const bool accept = ratio <= 1.0;
-  const double factor = fmin(FACTOR_MAX, fmax(0.2, 0.9 * pow(fmax(ratio, 1e-12), -1.0 / ERROR_ORDER)));
   double t_new = t[s];
   if (accept) {
     y[(size_t)i * ld + s] = y1;
     t_new += hs;
   }
   const double remaining = t_end - t_new;
-  double h_new = hs * (accept ? factor : fmin(factor, 0.5));
+  double h_new = next_step(hs, ratio, accept);
   if (i == 0) {
     t[s] = t_new;
     steps[s] += 1;
@@ -435,3 +456,132 @@ extern "C" __global__ void __launch_bounds__(256) rosenbrock_running(unsigned n,
 extern "C" __global__ void __launch_bounds__(64) rosenbrock_clear(unsigned* __restrict__ count) {
   if (threadIdx.x == 0) *count = 0u;
 }
+
+#ifdef WHOLE_STEPS
+// Whole steps of RODAS4, `count` at a time, for systems of at most 8 components: the right-hand side and the Jacobian
+// (reactor_rhs, reactor_jacobian: the same programs, compiled into this kernel) run on the first P lanes of the wave, one
+// system each, with inputs and outputs in LDS; the factors, stage vectors and step control stay in registers. A step of
+// separate kernels is 12 launches of 2 to 9 us each, nearly all of it latency; here it is one dependent chain.
+// 10^4 reactors of six species through ignition, 648 steps: 24.6 ms against 55.9 (38 us a step against 87); a step of 1000
+// takes 29 us, bound by the chain of programs, shuffles and LDS round trips. 256 registers a lane: the Jacobian program
+// would take more (it spills 52), but two waves a SIMD hide each other's latency.
+// Every operation and its rounding are those of the separate kernels. 
+#define IN (M + 1)
+#define OUT (M + M * M)
+
+// Stage I's right-hand side r = h f(Y_I) + Σ_{j<I} c_Ij k_j and the part of Y_{I+1} from the stages before I.
+template <int I>
+__device__ __forceinline__ void combine(double& r, double& z, const double (&k)[5]) {
+#pragma unroll
+  for (int j = 1; j < I; j++) {
+    r = __builtin_fma(rodas_c(I, j), k[j - 1], r);
+    if (I < 6) z = __builtin_fma(rodas_a(I + 1, j), k[j - 1], z);
+  }
+}
+
+extern "C" __global__ void __launch_bounds__(64, 2)
+rosenbrock_steps(int count, unsigned n, size_t ld, const double* __restrict__ P_in, double* __restrict__ y, double* __restrict__ t,
+                 double* __restrict__ h, int* __restrict__ status, unsigned* __restrict__ steps, double t_end, double rtol, double atol0,
+                 double atol) {
+  __shared__ double in[P][IN | 1], out[P][OUT | 1];
+  const int lane = threadIdx.x;
+  const int sys = lane / M, i = lane - sys * M, base = sys * M;
+  const bool row = sys < P;
+  const unsigned s = system_group() * P + (unsigned)(row ? sys : 0);
+  const bool valid = row && s < n;
+  const unsigned sv = valid ? s : 0u;
+  const bool mine = valid && status[sv] == 0;
+  bool active = mine;
+  const int ir = row ? i : 0;
+  double yi = row ? y[(size_t)ir * ld + sv] : 0.0, ti = t[sv], hi = h[sv];
+  int st = 0;
+  unsigned taken = 0;
+  const int at = i == 0 ? 0 : i + 1;  // T, P, Y_0..
+  if (row && i == 0) in[sys][1] = P_in[sv];
+  for (int step = 0; step < count; step++) {
+    const double left = t_end - ti;
+    if (active && left <= 1e-12 * fabs(t_end)) {
+      st = 1;
+      active = false;
+    }
+    if (__builtin_amdgcn_ballot_w64(active) == 0) break;  // uniform over the wave, which is the block
+    const double hs = fmin(hi, left);
+    if (active) hi = hs;
+    if (row) in[sys][at] = yi;
+    __syncthreads();
+    if (lane < P) reactor_jacobian(in[lane], out[lane]);
+    __syncthreads();
+    double a[M], k[5];
+    int perm[M];
+    int pos = -1;
+    const double f0 = row ? out[sys][ir] : 0.0;
+#pragma unroll
+    for (int j = 0; j < M; j++) {
+      const double Jij = row ? out[sys][M + ir * M + j] : 0.0;
+      a[j] = (row ? -hs * GAMMA * Jij : 0.0) + (row && i == j ? 1.0 : 0.0);
+    }
+    const double diag = factor(a, perm, pos, row, i, base);
+    const double rd = 1.0 / diag;
+    k[0] = solve(a, pos, perm, rd, GAMMA * hs * f0, i, base);
+#pragma unroll
+    for (int j = 1; j < 5; j++) k[j] = 0.0;
+    double ysi = __builtin_fma(rodas_a(2, 1), k[0], yi), x = 0.0;
+#pragma unroll 1
+    for (int stage = 2; stage <= 6; stage++) {
+      __syncthreads();
+      if (row) in[sys][at] = ysi;
+      __syncthreads();
+      if (lane < P) reactor_rhs(in[lane], out[lane]);
+      __syncthreads();
+      double r = row ? hs * out[sys][ir] : 0.0, z = row ? yi : 0.0;
+      switch (stage) {
+        case 2: combine<2>(r, z, k); break;
+        case 3: combine<3>(r, z, k); break;
+        case 4: combine<4>(r, z, k); break;
+        case 5: combine<5>(r, z, k); break;
+        default: combine<6>(r, z, k); break;
+      }
+      x = solve(a, pos, perm, rd, GAMMA * r, i, base);
+      switch (stage) {
+        case 2: k[1] = x; ysi = __builtin_fma(rodas_a(3, 2), x, z); break;
+        case 3: k[2] = x; ysi = __builtin_fma(rodas_a(4, 3), x, z); break;
+        case 4: k[3] = x; ysi = __builtin_fma(rodas_a(5, 4), x, z); break;
+        case 5: k[4] = x; ysi = __builtin_fma(rodas_a(6, 5), x, z); break;
+        default: break;
+      }
+    }
+    const double y1 = (row ? ysi : 0.0) + x;
+    const double ratio = error_ratio(x, row ? yi : 0.0, y1, row, i, base, rtol, atol0, atol);
+    const bool accept = ratio <= 1.0;
+    double t_new = ti;
+    if (accept) t_new += hs;
+    const double remaining = t_end - t_new;
+    double h_new = next_step(hs, ratio, accept);
+    if (active) {
+      if (accept) yi = y1;
+      ti = t_new;
+      taken++;
+      if (remaining <= 1e-12 * fabs(t_end)) {
+        st = 1;
+        active = false;
+      } else {
+        h_new = fmin(h_new, remaining);
+        if (h_new < H_MIN) {
+          st = 2;
+          active = false;
+        }
+        hi = h_new;
+      }
+    }
+    __syncthreads();
+  }
+  if (!mine) return;
+  y[(size_t)i * ld + s] = yi;
+  if (i == 0) {
+    t[s] = ti;
+    h[s] = hi;
+    steps[s] += taken;
+    status[s] = st;
+  }
+}
+#endif

@@ -200,7 +200,8 @@ void cb_cpu_module_free(cb_cpu_module* mod);
  * It stops after max_steps steps of the batch or when no reactor runs (found by a poll every 8 steps; the steps
  * launched before the host reads that poll leave every reactor alone and are not counted in *taken), and blocks
  * until then. Parts of the batch run on streams of the integrator's own, after the work already on `stream` and
- * joined back into it. An integrator keeps device buffers sized for its last batch (allocated again, after a device
+ * joined back into it; or, with RODAS4, the analytic Jacobian and at most 4096 waves of reactors of at most 8 state rows, whole
+ * steps run in one kernel on `stream`, with the same results to the bit. An integrator keeps device buffers sized for its last batch (allocated again, after a device
  * synchronization, when n, y, P or status change); calls on one integrator must not overlap. */
 enum cb_integrator_flags {
   CB_JACOBIAN_AUTOMATIC = 0,   /* the analytic program up to 8 state rows (K <= 7), difference quotients above */
