@@ -785,6 +785,8 @@ TransportPairs pairs_of(const ProgramView& p, int form_flags) {
   return transport_pairs(*p.mechanism, polynomials(p));
 }
 
+constexpr size_t kForkWork = size_t(1) << 27;  // states × species² from which two kernels of a call take two streams
+
 class Tiled : public SoAForm {
  public:
   // form 1: FP64 rates and transport; 2: MFMA mixed rates, FP32 transport; 3: FP32-core rates, FP32 transport.
@@ -829,7 +831,7 @@ class Tiled : public SoAForm {
   // after the other instead: up to kForkWork (48 k states of 53 species, where they take 45 us each; 4096 states of 10
   // species, 8 us each, take 15 instead of 41 us), except for the large-mechanism and MFMA rates kernels, whose
   // smallest batches already take 50 us from 32 species on.
-  static constexpr size_t kForkWork = size_t(1) << 27, kForkSpecies = 32;
+  static constexpr size_t kForkSpecies = 32;
   void launch(const double* const* in, double* const* out, size_t n, const Launch& how) override {
     hipStream_t stream = how.stream;
     const bool slow = (mixed_ || tiled_rates_) && species_ >= kForkSpecies;
@@ -889,6 +891,17 @@ std::string surrogate_text(int K, const MlpLayout& lay, int DK, int NM) {
 // FP32-core straight-line rates (or the MFMA mixed rates), then the transport surrogate with the plain FP64 transport
 // kernel on the states outside its box.
 class Surrogate : public SoAForm {
+  // The weights of every layer in the order of the kernel's loads, lane by lane: 16 rows × 32 inputs after each other, of
+  // which lane 16 (i mod 32 / 8) + o mod 16 takes 8 inputs.
+  static std::vector<uint16_t> fragments(const std::vector<uint16_t>& w, const MlpLayout& lay) {
+    std::vector<uint16_t> f(w);
+    for (const auto& L : lay.layers)
+      for (long o = 0; o < L.out; o++)
+        for (long i = 0; i < L.in; i++)
+          f[L.w + ((o / 16 * (L.in / 32) + i / 32) * 64 + i % 32 / 8 * 16 + o % 16) * 8 + i % 8] = w[L.w + o * L.in + i];
+    return f;
+  }
+
  public:
   Surrogate(const ProgramView& p, const SurrogateWeights& w) : SoAForm(p.function->n_input, (int)p.function->output.size()) {
     check_program(p);
@@ -958,7 +971,7 @@ class Surrogate : public SoAForm {
     }
     kernel_.load(device::compile(surrogate_text(K, lay, DK, NM), "surrogate_transport", hip_options(true)), "surrogate_transport");
     device::check(hipModuleGetFunction(&clear_, kernel_.module, "surrogate_clear"), "hipModuleGetFunction surrogate_clear");
-    d_w16_ = upload(to_bf16(w.params));
+    d_w16_ = upload(fragments(to_bf16(w.params), lay));
     d_params_ = upload(w.params);
     d_offsets_ = upload(offsets);
     d_f_mean_ = upload(w.f_mean);
@@ -1015,9 +1028,12 @@ class Surrogate : public SoAForm {
       list = d_fallback_;
     }
     // The rates kernel on the caller's stream; the surrogate and its fallback on a side stream forked from and joined
-    // back into it (the two read the same inputs and write disjoint outputs), as in the tiled forms.
+    // back into it (the two read the same inputs and write disjoint outputs), as in the tiled forms and from as many
+    // states on (53 species, forked against one after the other: 2^18 states 593 against 695 us, 2^16 228 against 244,
+    // 20000 145 against 129).
     hipStream_t ts = stream;
-    const bool fork = (rates_ || mixed_) && !how.single_stream;
+    const size_t K = (size_t)n_inputs() - 2;
+    const bool fork = (mixed_ || (rates_ && n >= kForkWork / (K * K))) && !how.single_stream;
     if (fork) {
       if (!side_) {
         device::check(hipStreamCreateWithFlags(&side_, hipStreamNonBlocking), "hipStreamCreateWithFlags");
