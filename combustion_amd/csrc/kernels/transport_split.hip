@@ -106,7 +106,7 @@ transport_fp64(const double* const* __restrict__ in, double* const* __restrict__
     mass += lds_s[(2 * WAVES + w) * 64 + lane];
   }
   const double density = C_tot * rcp64(sum), bulk = C_tot - density * positive;
-  const double WN = density * mass + W[K - 1] * bulk;  // Σ W_k x_k
+  const double WN = __builtin_fma(W[K - 1], bulk, density * mass);  // Σ W_k x_k
   __syncthreads();
   double v[KW], A = 0.0, B = 0.0;
 #pragma unroll
@@ -155,8 +155,8 @@ transport_fp64(const double* const* __restrict__ in, double* const* __restrict__
     const int k = wave + WAVES * i;
     if (k < K) {
       x[i] = X(k);
-      const double den = d0[i] + v[i] * (2.0 * d1[i] + v[i] * d2[i]);
-      mu += x[i] * (v[i] * v[i]) * rcp64(den);
+      const double den = __builtin_fma(v[i], __builtin_fma(v[i], d2[i], 2.0 * d1[i]), d0[i]);
+      mu = __builtin_fma(x[i] * (v[i] * v[i]), rcp64(den), mu);
     }
   }
   __syncthreads();

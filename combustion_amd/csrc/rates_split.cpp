@@ -426,13 +426,14 @@ void replace(std::string& text, const std::string& what, const std::string& with
 
 }  // namespace
 
-RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast) {
+RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast, bool one_team) {
   const size_t K = m.species.len(), KA = m.active;
   RatesSplit t;
   // Eight waves per CU (two per SIMD, 256 registers each): two teams of four waves where their LDS fits (up to 53
   // species with one of them inert), since each part pays for the shared prologue and the sums, else one team of eight.
   t.teams = (2 * KA + K) * 128 * sizeof(double) <= 160 * 1024 ? 2 : 1;
   t.parts = 8 / t.teams;
+  if (one_team) t.teams = 1;
   Writer w(m, fast);
   // Sections: the longest reaction first, each to the part with the least work so far.
   const size_t R = m.reactions.size();
@@ -480,7 +481,7 @@ RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast) {
   head << "#define NAME " << name << "\n#define K " << K << "\n#define KA " << KA << "\n#define PARTS " << t.parts << "\n#define TEAMS " << t.teams
        << "\n#define FAST " << (fast ? 1 : 0) << "\n";
   t.source = head.str() + rates_split_source;
-  replace(t.source, "@LDS_V@", std::to_string(std::max({KA * 256, (size_t)(t.teams == 1 ? (2 * KA + K) * 64 : 0), (size_t)1024})));
+  replace(t.source, "@LDS_V@", std::to_string(std::max({KA * 32 * (size_t)(t.parts * t.teams), (size_t)(t.teams == 1 ? (2 * KA + K) * 64 : 0), (size_t)1024})));
   replace(t.source, "@SECTIONS@\n", s.str());
   replace(t.source, "@STORE@\n", store.str());
   replace(t.source, "@ADD@\n", add.str());

@@ -15,6 +15,7 @@ struct RatesSplit {
 };
 
 // fast: exponentials and logarithms on the FP32 cores (CB_FORM_FAST). Mechanisms of up to 64 species.
-RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast);
+// one_team: a team of four waves alone in its block, for mechanisms that otherwise run two.
+RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast, bool one_team = false);
 
 }  // namespace combustion

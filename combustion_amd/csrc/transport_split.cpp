@@ -169,6 +169,11 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
     for (size_t i = 0; kWaves * i + wave < K; i++) v.push_back((int)i);
     return v;
   };
+  // sum = or += c x, the operation spelt out: which of the first two products of a sum contraction rounds depends on the
+  // text around it, and this text is also part of another kernel (rates_and_transport), with the same results
+  auto term = [](const std::string& sum, const std::string& c, const std::string& x, bool first) {
+    return "    " + sum + " = " + (first ? c + " * " + x : "__builtin_fma(" + c + ", " + x + ", " + sum + ")") + ";\n";
+  };
   std::vector<std::string> columns, rows, own, next, half;
   for (int w = 0; w < kWaves; w++) {
     // Gᵀ y_m for the columns w, w + 4, ..; four species to a block
@@ -181,7 +186,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
         for (size_t i = 0; kWaves * i + w < R; i++) {
           const std::string c = literal(G[j * R + kWaves * i + w] * std::sqrt(W[j] / 8.));
           for (int mth = 0; mth < 3; mth++)
-            text << "    z[" << i << "][" << mth << "] " << (j ? "+= " : "= ") << c << " * " << (mth == 0 ? "x" + std::to_string(j) : "y" + std::to_string(mth)) << ";\n";
+            text << term("z[" + std::to_string(i) + "][" + std::to_string(mth) + "]", c, mth == 0 ? "x" + std::to_string(j) : "y" + std::to_string(mth), j == 0);
         }
         text << "  }\n";
       }
@@ -196,7 +201,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
       for (int i : slots(w)) {
         const size_t k = kWaves * i + w;
         const std::string c = literal(G[k * R + q] / std::sqrt(W[k]));
-        for (int mth = 0; mth < 3; mth++) text << "  d" << mth << "[" << i << "] " << (q ? "+= " : "= ") << c << " * z" << q << "_" << mth << ";\n";
+        for (int mth = 0; mth < 3; mth++) text << term("d" + std::to_string(mth) + "[" + std::to_string(i) + "]", c, "z" + std::to_string(q) + "_" + std::to_string(mth), q == 0);
       }
       r.add(read.str(), text.str());
     }
