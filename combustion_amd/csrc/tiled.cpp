@@ -666,7 +666,7 @@ class RatesStraight {
                                         t_.split.parts ? teams : straight, nullptr),
                   "launch rates");
   }
-  bool teams_of_four() const { return t_.split.parts == 4; }
+  const RatesText& text() const { return t_; }
   double *const& rcp_W() const { return d_rcp_W_; }
   double *const& gibbs() const { return d_gibbs_; }
 
@@ -758,9 +758,9 @@ class TransportStraight {
 
 // A kernel's text as the device function `space`::run, its block index the first argument; its macros end with it.
 std::string as_function(std::string text, const std::string& kernel, const std::string& space) {
-  const size_t from = text.find("extern \"C\" __global__"), to = from == std::string::npos ? from : text.find("\n" + kernel + "(", from);
+  const size_t from = text.find("extern \"C\" __global__"), to = from == std::string::npos ? from : text.find(kernel + "(", from);
   if (to == std::string::npos) throw std::logic_error("no kernel " + kernel + " in its text");
-  text.replace(from, to + kernel.size() + 2 - from, "__device__ __forceinline__ void run(const unsigned block, ");
+  text.replace(from, to + kernel.size() + 1 - from, "__device__ __forceinline__ void run(const unsigned block, ");
   for (size_t at; (at = text.find("blockIdx.x")) != std::string::npos;) text.replace(at, 10, "block");
   std::string ends;
   std::istringstream lines(text);
@@ -769,45 +769,64 @@ std::string as_function(std::string text, const std::string& kernel, const std::
   return "namespace " + space + " {\n" + text + "\n}\n" + ends;
 }
 
-// The team kernels of both sections in one launch, a block of either's 256 threads over 64 states.
-std::string rates_and_transport_text(const ProgramView& p, const TransportText& transport) {
-  const RatesSplit rates = rates_split(*p.mechanism, "rates_fp64", false, true);
-  return as_function(rates.source, "NAME", "rates") + as_function(transport.source, "transport_fp64", "transport") +
-         "extern \"C\" __global__ void __launch_bounds__(256, 2)\n"
-         "rates_and_transport(const double* const* __restrict__ in, double* const* __restrict__ out, double* const* __restrict__ tout,\n"
-         "                    unsigned n, unsigned groups, const double* __restrict__ rcp_W, const double* __restrict__ gibbs,\n"
-         "                    double clamp_pos, double clamp_neg, const double* __restrict__ W, const double* __restrict__ fit_c,\n"
-         "                    const double* __restrict__ fit_v, double rcp_T0) {\n"
-         "  if (blockIdx.x < groups)\n"
-         "    transport::run(blockIdx.x, in, tout, n, rcp_W, W, fit_c, fit_v, rcp_T0);\n"
-         "  else\n"
-         "    rates::run(blockIdx.x - groups, in, out, n, rcp_W, gibbs, clamp_pos, clamp_neg);\n"
-         "}\n";
+// Both sections in one launch: the team kernels, a block of either's 256 threads over 64 states, or the one-lane kernels in
+// blocks of one wave.
+std::string rates_and_transport_text(const ProgramView& p, const RatesText& r, const TransportText& transport) {
+  const bool teams = r.split.parts != 0;
+  const std::string rates = teams ? rates_split(*p.mechanism, "rates_fp64", false, true).source : r.source;
+  std::ostringstream s;
+  s << as_function(rates, teams ? "NAME" : "rates_fp64", "rates") << as_function(transport.source, "transport_fp64", "transport")
+    << "extern \"C\" __global__ void __launch_bounds__(" << (teams ? "256, 2" : "64")
+    << ")\n"
+       "rates_and_transport(const double* const* __restrict__ in, double* const* __restrict__ out, double* const* __restrict__ tout,\n"
+       "                    unsigned n, unsigned groups, const double* __restrict__ rcp_W, const double* __restrict__ gibbs,\n"
+       "                    double clamp_pos, double clamp_neg, const double* __restrict__ W, const double* __restrict__ fit_c,\n"
+       "                    const double* __restrict__ fit_v, double rcp_T0) {\n"
+       "  if (blockIdx.x < groups)\n"
+       "    transport::run(blockIdx.x, in, tout, n, "
+    << (teams ? "rcp_W, W, fit_c, fit_v, rcp_T0" : "0u")
+    << ");\n"
+       "  else\n"
+       "    rates::run(blockIdx.x - groups, in, out, n, "
+    << (teams ? "rcp_W, gibbs, clamp_pos, clamp_neg" : "0u") << ");\n}\n";
+  return s.str();
+}
+
+// The FP64 kernels that one launch may run both of: teams of four waves in both sections (32 to 53 species: two teams'
+// LDS is 160 KB there), or one lane per state in both.
+bool one_launch(const RatesText& r, const TransportText& t) {
+  const bool split = !t.split.W.empty();
+  return r.split.parts == 4 ? split : r.split.parts == 0 && !split;
 }
 
 // Both sections of a small batch in one kernel: their blocks run beside each other, where two launches on one stream run
-// one after the other and two streams cost more to fork and join than either kernel takes. 53 species, 1 to 8192 states: 30 to 33 us against 54 to
-// 57. The same operations as the two kernels', and so the same results.
-// One block a CU (both sections' LDS counts, 134 KB at 53 species), so for batches whose blocks are at most the chip's CUs.
+// one after the other and two streams cost more to fork and join than either kernel takes. 53 species, 1 to 8192 states:
+// 30 to 33 us against 54 to 57; 10 species 10 against 14.5, 24 species 24 against 43 (4096 states). The same operations as
+// the two kernels', and so the same results.
+// Team kernels: one block a CU (both sections' LDS counts, 134 KB at 53 species), so for batches whose blocks are at most
+// the chip's CUs. One lane per state: every size, since large batches fill the chip better from one launch than from two
+// streams (10 species, 2^20 states: 121 against 131 us; 24 species, 2^19: 275 against 290).
 class RatesAndTransport {
  public:
-  static constexpr size_t kStates = 64 * 128;
-  // FP64 teams of four waves in both sections (at most 53 species: two teams' LDS is 160 KB there).
-  static bool applies(const RatesStraight& r, const TransportStraight& t) { return r.teams_of_four() && t.split(); }
-  RatesAndTransport(const ProgramView& p, const RatesStraight& r, const TransportStraight& t) : r_(r), t_(t) {
-    kernel_.load(device::compile(rates_and_transport_text(p, t.text()), "rates_and_transport", hip_options(true)), "rates_and_transport");
+  static constexpr size_t kTeamStates = 64 * 128;
+  RatesAndTransport(const ProgramView& p, const RatesStraight& r, const TransportStraight& t) : r_(r), t_(t), teams_(r.text().split.parts != 0) {
+    kernel_.load(device::compile(rates_and_transport_text(p, r.text(), t.text()), "rates_and_transport", hip_options(true)),
+                 "rates_and_transport");
   }
+  bool takes(size_t n) const { return !teams_ || n <= kTeamStates; }
   void launch(const double* const* in, double* const* out, double* const* tout, size_t n, hipStream_t stream) {
     unsigned n32 = (unsigned)n, groups = (unsigned)((n + 63) / 64);
     double pos = 6981463048192., neg = (double)cbrtf(3.40282347e38f);  // reaction.rs:244-256
     double *rcp_W = r_.rcp_W(), *gibbs = r_.gibbs(), *W = t_.d_W_, *c = t_.d_c_, *v = t_.d_v_, rcp_T0 = t_.rcp_T0_;
     void* args[] = {&in, &out, &tout, &n32, &groups, &rcp_W, &gibbs, &pos, &neg, &W, &c, &v, &rcp_T0};
-    device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, 256, 1, 1, 0, stream, args, nullptr), "launch rates_and_transport");
+    device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, teams_ ? 256 : 64, 1, 1, 0, stream, args, nullptr),
+                  "launch rates_and_transport");
   }
 
  private:
   const RatesStraight& r_;
   const TransportStraight& t_;
+  bool teams_;
   device::Kernel kernel_;
 };
 
@@ -874,7 +893,7 @@ class Tiled : public SoAForm {
       else
         transport_ = std::make_unique<TransportTiled>(p, f64);
     }
-    if (f64 && fp64_ && straight_ && RatesAndTransport::applies(*fp64_, *straight_))
+    if (f64 && fp64_ && straight_ && one_launch(fp64_->text(), straight_->text()))
       small_ = std::make_unique<RatesAndTransport>(p, *fp64_, *straight_);
   }
 
@@ -890,13 +909,12 @@ class Tiled : public SoAForm {
   // caller's stream, so that the two kernels' blocks share the CUs (1.74 against 1.76 ms per 2^20 states at K=53; 4096
   // states of 160 species in the mixed form, whose few blocks leave most of the chip idle, 0.37 against 0.53 ms). The
   // fork and join take about 25 us on the GPU and 15 us of the host's time, so that kernels of that length run in one
-  // launch where there is a kernel for both, and one after the other else: up to kForkWork (48 k states of 53 species, where they take 45 us each; 4096 states of 10
-  // species, 8 us each, take 15 instead of 41 us), except for the large-mechanism and MFMA rates kernels, whose
+  // launch where there is a kernel for both, and one after the other else: up to kForkWork (48 k states of 53 species, where they take 45 us each), except for the large-mechanism and MFMA rates kernels, whose
   // smallest batches already take 50 us from 32 species on.
   static constexpr size_t kForkSpecies = 32;
   void launch(const double* const* in, double* const* out, size_t n, const Launch& how) override {
     hipStream_t stream = how.stream;
-    if (small_ && n <= RatesAndTransport::kStates) return small_->launch(in, out, out + n_rates_, n, stream);
+    if (small_ && small_->takes(n)) return small_->launch(in, out, out + n_rates_, n, stream);
     const bool slow = (mixed_ || tiled_rates_) && species_ >= kForkSpecies;
     const bool both = (mixed_ || fp64_ || tiled_rates_) && (straight_ || transport_ || pairs_) && !how.single_stream &&
                       (slow || n >= kForkWork / (species_ * species_));
@@ -1191,8 +1209,10 @@ void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
     else if (straight_transport(p, form_flags)) {
       const TransportText t = transport_text(p, !mixed);
       device::compile(t.source, t.name, hip_options(true));
-      if (p.chemistry->options.rates && !mixed && !tiled_rates(p, form_flags) && !t.split.W.empty() && rates_text(p, false).split.parts == 4)
-        device::compile(rates_and_transport_text(p, t), "rates_and_transport", hip_options(true));
+      if (p.chemistry->options.rates && !mixed && !tiled_rates(p, form_flags)) {
+        const RatesText r = rates_text(p, false);
+        if (one_launch(r, t)) device::compile(rates_and_transport_text(p, r, t), "rates_and_transport", hip_options(true));
+      }
     }
     else
       device::compile(transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed), "transport_tiled",

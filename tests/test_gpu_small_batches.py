@@ -43,3 +43,27 @@ def test_small_batches_equal_larger_ones(species, D, gpu):
             g.replay()
             torch.cuda.synchronize()
             assert torch.equal(torch.stack(outs), whole[:, :n]), (species, n)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("species", [10, 24])
+def test_one_lane_kernels_in_one_launch(species, gpu):
+    """Mechanisms whose two sections run one lane per state, at every size in one launch of blocks of 64 states: 1e-12 of
+    the oracle, and nothing written past the batch."""
+    import torch
+    if species == 10:
+        M, mech, o = setup("h2o2-10")
+    else:
+        M, mech, o = setup_text(synth.generate(24, 120, 6, 4, 24, "small-24").yaml())
+    mod = M.chemistry().assemble(form="fp64")
+    T, P, Y = synth.states(M.K, 333, 5, (300.0, 3000.0), (0.1, 50.0), 0.3)
+    ref, floor = o.batch(T, P, Y, threads=8)
+    for n in (1, 63, 64, 65, 256, 257, 333):
+        ins = [torch.from_numpy(np.ascontiguousarray(x[:n])).to(gpu) for x in (T, P, *Y)]
+        room = torch.full((len(ref), n + 1), float("nan"), dtype=torch.float64, device=gpu)
+        mod(ins, [x[:n] for x in room])
+        torch.cuda.synchronize()
+        assert room[:, n].isnan().all()
+        err = relative_error(room[:, :n].cpu().numpy(), ref[:, :n], np.abs(floor[:, :n])).max()
+        print(species, n, err, flush=True)
+        assert err < 1e-12
