@@ -20,6 +20,9 @@ extern const char* const rosenbrock_source;
 
 namespace {
 constexpr int kPollEvery = 8;
+// Reactors of a large mechanism up to which the batch is one part (53 species, us a step, one part against four: 100
+// reactors 591 against 695, 1000 661 against 726, 4000 934 against 922, 16000 2197 against 2161).
+constexpr size_t kOnePart = 2048;
 // Waves of rosenbrock_steps up to which it is faster than the separate kernels: its programs use one lane in seven, so
 // that beyond four waves a SIMD the chip is busy with them (six species, us a step, whole against separate: 1000 reactors
 // 29 against 86, 10^4 38 against 87, 2·10^4 57 against 88, 5·10^4 101 against 99, 2·10^5 349 against 260).
@@ -204,6 +207,10 @@ void Integrator::release() {
   last_status_ = nullptr;
 }
 
+// Large mechanisms in small batches run as one part: a step is then a chain of launches that leave most of the chip idle
+// however many parts share it, and one part can run the two right-hand sides of its Jacobian beside each other.
+size_t Integrator::parts_of(size_t n) const { return differences_ && m_ > 32 && n <= kOnePart ? 1 : parts_count_; }
+
 // What the polls of either path need: the events and the pinned words behind which the running counts arrive.
 void Integrator::prepare_polls() {
   if (host_count_) return;
@@ -249,7 +256,7 @@ void Integrator::prepare(double* y, const double* P, const int* status, size_t n
     raised_T_ = (double*)alloc(n * sizeof(double));
   }
   // the batch in parts_count_ parts, each on its own stream, each starting at a multiple of 8 reactors (64-byte rows)
-  const int parts = parts_count_;
+  const int parts = (int)parts_of(n);
   std::vector<size_t> bounds;
   for (int k = 0; k <= parts; k++) bounds.push_back(k == parts ? n : std::min(n, (n * k / parts + 7) & ~(size_t)7));
   auto table = [&](const std::vector<const void*>& ptrs) {
@@ -397,9 +404,20 @@ long Integrator::advance(double* y, const double* P, double* t, double* h, int* 
         const size_t fields = count * 2 * m;
         device::check(hipModuleLaunchKernel(copies_kernel, (unsigned)((fields + 255) / 256), 1, 1, 256, 1, 1, 0, st, rargs, nullptr),
                       "launch rosenbrock_copies");
+        // in one part, the right-hand side at the raised temperature runs beside that of the copies
+        hipStream_t beside = parts_.size() == 1 ? sides_[0] : st;
+        if (beside != st) {
+          device::check(hipEventRecord(fork_, st), "hipEventRecord");
+          device::check(hipStreamWaitEvent(beside, fork_, 0), "hipStreamWaitEvent");
+          rhs_->launch_only((const double* const*)q.tab_t_in, (double* const*)q.tab_t_out, count, beside, nullptr);
+          device::check(hipEventRecord(join_, beside), "hipEventRecord");
+        }
         shared_->launch_only((const double* const*)q.tab_shared_in, (double* const*)q.tab_shared_out, count, st, nullptr);
         varying_->launch_only((const double* const*)q.tab_rep_in, (double* const*)q.tab_rep_out, count * C, st, nullptr);
-        rhs_->launch_only((const double* const*)q.tab_t_in, (double* const*)q.tab_t_out, count, st, nullptr);
+        if (beside != st)
+          device::check(hipStreamWaitEvent(st, join_, 0), "hipStreamWaitEvent");
+        else
+          rhs_->launch_only((const double* const*)q.tab_t_in, (double* const*)q.tab_t_out, count, st, nullptr);
       } else {
         jacobian_->launch_only((const double* const*)q.tab_y, (double* const*)q.tab_jac, count, st, nullptr);
       }

@@ -46,7 +46,7 @@ class Integrator {
   double rtol_, atol_T_, atol_Y_;
   bool differences_;
   int phases_;  // Rosenbrock phases per step: 3 (ode23s) or 6 (RODAS4)
-  int parts_count_;  // the batch's parts, each on its own stream
+  int parts_count_;  // the most parts of a batch, each on its own stream
   unsigned systems_per_wave_;
   ast::Function rhs_function_, jacobian_function_, shared_function_, varying_function_;
   ast::Linear rhs_linear_, jacobian_linear_, shared_linear_, varying_linear_;
@@ -58,7 +58,7 @@ class Integrator {
   int* perm_ = nullptr;
   unsigned* running_ = nullptr;
   double *groups_ = nullptr, *raised_T_ = nullptr;  // each reactor's values for its copies; the raised temperatures
-  // The batch runs in parts_count_ parts, the first on the caller's stream and the others on sides_, so that one
+  // The batch runs in one part or parts_count_, the first on the caller's stream and the others on sides_, so that one
   // part's latency-bound right-hand sides overlap another's Rosenbrock phases. Each part's pointer tables start at its
   // first reactor: the programs' inputs from y or ys and outputs to F or jac; for difference quotients, the shared
   // part's inputs [T, P] and outputs, the copies' inputs (the reactors' values and status) and outputs, and the
@@ -82,6 +82,7 @@ class Integrator {
   const int* last_status_ = nullptr;
   void release();
   void prepare(double* y, const double* P, const int* status, size_t n);
+  size_t parts_of(size_t n) const;
   void prepare_polls();
   void join_sides(hipStream_t stream);
   bool poll(unsigned* running, const int* status, unsigned n, long taken, hipStream_t stream, hipFunction_t clear, hipFunction_t count_running,
