@@ -12,7 +12,7 @@
 //   3. the parts' sums, in a fixed order: the upper half of the parts hands its sums to the lower half through LDS,
 //      then every part adds the rows of its own species and writes them out
 //
-// Bound: FP64 VALU issue. Per 64 states of the 53-species mechanism it issues 16.5 k VALU instructions where the
+// Bound: FP64 VALU issue. Per 64 states of the 53-species mechanism it issues 17.3 k VALU instructions where the
 // one-lane kernel issued 23.4 k (no accumulation-register moves, base-2 exponentials without clamps of their own, one
 // exponential per rate constant, one factor per product species) at one wave per SIMD; with two waves per SIMD and the
 // parts' scalar constants and LDS reads beside the other wave's arithmetic, 2^20 states take 0.80 ms against 1.19 ms,

@@ -41,15 +41,15 @@ enum cb_status {
 /* Program forms for cb_hip_assemble. */
 enum cb_form {
   CB_FORM_STRAIGHT = 0, /* the program emitted as straight-line HIP, one lane per state (cuda.rs:101-134) */
-  CB_FORM_FP64 = 1,     /* chemistry programs: FP64 rates and transport sections as separate kernels (straight-line rates
-                           and transport up to 64 species; the table-driven rates kernel and the tiled MFMA transport
-                           kernel above) */
+  CB_FORM_FP64 = 1,     /* chemistry programs: FP64 rates and transport sections as separate kernels, or one kernel for both (up
+                           to 64 species generated code, one lane per state or teams of waves; above, the table-driven
+                           rates kernel and the transport kernel of sixteen waves, beyond 160 species of MFMA tiles) */
   CB_FORM_MIXED = 2,    /* tiled mixed precision: BF16-split MFMA contractions, FP32 exp/log, FP64 ΔG/RT */
   CB_FORM_FAST = 3      /* FP64 straight-line rates with FP32 cores for exp and ln, FP32 transport */
 };
 /* Modifier ORed into the form of a chemistry program (forms 1-3): the transport section takes the tiled MFMA
  * kernel (Wilke sums and binary-diffusion polynomials as v_mfma_{f64,f32}_16x16x4 contractions) at any species
- * count, instead of the straight-line transport kernel that forms 1 and 3 use up to 64 species. */
+ * count, instead of the transport kernels that forms 1 and 3 use up to 64 species, and form 1 up to 160. */
 enum cb_form_flags { CB_FORM_TILED_TRANSPORT = 0x10,
 /* Modifier for forms 1 and 3: the rates section takes the table-driven FP64 kernel (8 states x 8 reaction groups per
  * wave, per-state arrays in LDS) that those forms use above 64 species, instead of the straight-line rates kernel. */
