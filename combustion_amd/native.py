@@ -434,6 +434,8 @@ class Module:
             optrs = [_pointer(x) for x in outputs]
             if any(d != on_device for _, d in optrs) or len(outputs) != n_out:
                 raise ValueError("outputs must match the inputs' placement and the program's output count")
+            if any((x.size if isinstance(x, np.ndarray) else x.numel()) < n for x in outputs):
+                raise ValueError(f"outputs must have room for all {n} states")
             out_arr[:] = [p for p, _ in optrs]
         ms = C.c_float(0)
         _check(lib().cb_hip_call(self._h, in_arr, n_in, n, out_arr, n_out, int(on_device), stream,
