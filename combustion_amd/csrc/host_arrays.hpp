@@ -99,7 +99,7 @@ class HostArrays {
     return true;
   }
 
-  // run(din, n, dout, stream) launches the module's kernels on device arrays, on `stream`.
+  // run(slot, din, n, dout, stream) launches the module's kernels on a slot's device arrays, on `stream`.
   template <class Run>
   void call(const double* const* inputs, size_t n, double* const* outputs, Run&& run) {
     const size_t rows = (size_t)(n_in_ + n_out_);
@@ -141,7 +141,7 @@ class HostArrays {
       for (int i = 0; i < n_out_; i++) dout[i] = s.device + (n_in_ + i) * per;
       team.run(n_in_, [&](int i) { std::memcpy(s.pinned + i * per, inputs[i] + first, count * sizeof(double)); });
       device::check(hipMemcpyAsync(s.device, s.pinned, n_in_ * per * sizeof(double), hipMemcpyHostToDevice, s.stream), "hipMemcpyAsync H2D");
-      run(din.data(), count, dout.data(), s.stream);
+      run((int)(slice % 2), din.data(), count, dout.data(), s.stream);
       device::check(hipMemcpyAsync(s.pinned + n_in_ * per, s.device + n_in_ * per, n_out_ * per * sizeof(double), hipMemcpyDeviceToHost, s.stream),
                     "hipMemcpyAsync D2H");
     }

@@ -17,6 +17,7 @@ class SoAForm : public Form {
   SoAForm(int n_inputs, int n_outputs) : n_in_(n_inputs), n_out_(n_outputs) {}
   ~SoAForm() override {
     for (void* slab : slabs_) (void)hipFree(slab);
+    for (const StagingTable& t : staging_) (void)hipFree(t.table);
     if (start_) (void)hipEventDestroy(start_);
     if (stop_) (void)hipEventDestroy(stop_);
     if (done_) (void)hipEventDestroy(done_);
@@ -35,9 +36,9 @@ class SoAForm : public Form {
       if (!host_) host_ = std::make_unique<HostArrays>(n_in_, n_out_);
       if (work_bytes(n) == 0 && host_->sliceable(inputs, n, outputs)) {
         if (kernel_ms) *kernel_ms = 0;
-        host_->call(inputs, n, outputs, [&](const double* const* din, size_t count, double* const* dout, hipStream_t slot) {
+        host_->call(inputs, n, outputs, [&](int slot, const double* const* din, size_t count, double* const* dout, hipStream_t slot_stream) {
           float ms = 0;
-          run(din, count, dout, slot, kernel_ms ? &ms : nullptr);
+          run(staging_table(staging_[slot], pointer_set(din, dout)), count, slot_stream, kernel_ms ? &ms : nullptr);
           if (kernel_ms) *kernel_ms += ms;
         });
         return;
@@ -56,14 +57,14 @@ class SoAForm : public Form {
         device::check(hipMemcpy(din[i], inputs[i], n * sizeof(double), hipMemcpyHostToDevice), "hipMemcpy H2D");
       }
       for (int i = 0; i < n_out_; i++) device::check(hipMalloc(&dout[i], n * sizeof(double)), "hipMalloc");
-      run(din.data(), n, dout.data(), stream, kernel_ms);
+      run(table_for(pointer_set(din.data(), dout.data())), n, stream, kernel_ms);
       device::check(hipStreamSynchronize(stream), "hipStreamSynchronize");
       forget_table(din.data(), dout.data());  // the staging arrays are freed on return
       for (int i = 0; i < n_out_; i++)
         device::check(hipMemcpy(outputs[i], dout[i], n * sizeof(double), hipMemcpyDeviceToHost), "hipMemcpy D2H");
       return;
     }
-    run(inputs, n, outputs, stream, kernel_ms);
+    run(table_for(pointer_set(inputs, outputs)), n, stream, kernel_ms);
   }
 
  protected:
@@ -139,6 +140,24 @@ class SoAForm : public Form {
     return table;
   }
 
+  // A staging slot's table, rewritten when the size of a call's slices moves the slot's arrays: every launch of the call
+  // before has completed, no graph is captured on host arrays, and the tables of the callers' own arrays stay untouched.
+  struct StagingTable {
+    void* table = nullptr;
+    std::vector<const void*> ptrs;
+  };
+  StagingTable staging_[2];
+
+  void* staging_table(StagingTable& t, std::vector<const void*> ptrs) {
+    if (!t.table) device::check(hipMalloc(&t.table, ptrs.size() * sizeof(void*)), "hipMalloc table");
+    if (t.ptrs != ptrs) {
+      t.ptrs.clear();
+      device::check(hipMemcpy(t.table, ptrs.data(), ptrs.size() * sizeof(void*), hipMemcpyHostToDevice), "hipMemcpy table");
+      t.ptrs = std::move(ptrs);
+    }
+    return t.table;
+  }
+
   std::vector<const void*> pointer_set(const double* const* inputs, double* const* outputs) const {
     std::vector<const void*> ptrs;
     for (int i = 0; i < n_in_; i++) ptrs.push_back(inputs[i]);
@@ -154,8 +173,7 @@ class SoAForm : public Form {
     tables_.erase(it);
   }
 
-  void run(const double* const* inputs, size_t n, double* const* outputs, hipStream_t stream, float* kernel_ms) {
-    void* table = table_for(pointer_set(inputs, outputs));
+  void run(void* table, size_t n, hipStream_t stream, float* kernel_ms) {
     auto in = (const double* const*)table;
     auto out = (double* const*)((const void**)table + n_in_);
     order_after_previous_call(stream);

@@ -1,0 +1,66 @@
+"""Calls on host arrays (csrc/host_arrays.hpp) and the pointer tables of csrc/soa.hpp, run on the CPU: host_calls.cpp puts
+the plumbing over HIP functions on host memory."""
+import ctypes as C
+import os
+import subprocess
+
+import numpy as np
+import pytest
+
+from combustion_amd.build import CSRC, ROCM
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+SLOT = (16 << 20) // (4 * 8)  # states of a slice of two inputs and two outputs
+
+
+@pytest.fixture(scope="module")
+def lib(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("host_calls") / "host_calls.so")
+    subprocess.check_call(["g++", "-O1", "-std=c++17", "-fPIC", "-shared", "-pthread", "-D__HIP_PLATFORM_AMD__", "-I" + CSRC,
+                           "-I" + os.path.join(ROCM, "include"), os.path.join(HERE, "host_calls.cpp"), "-o", so])
+    l = C.CDLL(so)
+    l.form_new.restype = C.c_void_p
+    l.form_launches.restype = C.c_size_t
+    l.form_launches.argtypes = l.form_free.argtypes = [C.c_void_p]
+    l.form_replay.argtypes = [C.c_void_p, C.c_size_t]
+    l.form_call.argtypes = [C.c_void_p, C.POINTER(C.c_void_p), C.c_size_t, C.POINTER(C.c_void_p), C.c_int, C.c_void_p]
+    l.queue_copy.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
+    return l
+
+
+class Form:
+    def __init__(self, lib):
+        self.lib, self.form = lib, lib.form_new()
+
+    def __del__(self):
+        self.lib.form_free(self.form)
+
+    def __call__(self, ins, outs, n=None, on_device=False, stream=None):
+        table = lambda arrays: (C.c_void_p * 2)(*[a.ctypes.data for a in arrays])
+        self.lib.form_call(self.form, table(ins), len(ins[0]) if n is None else n, table(outs), int(on_device), stream)
+        return self.lib.form_launches(self.form) - 1
+
+
+def states(n, seed=1):
+    return list(np.random.default_rng(seed).standard_normal((2, n)))
+
+
+def results(a, b):
+    return [a + b, a * b]
+
+
+def test_host_calls_leave_the_tables_of_captured_launches(lib):
+    """Host calls of more sizes than a module has pointer tables: a launch captured before them still has its own."""
+    form = Form(lib)
+    ins, outs = states(100), list(np.zeros((2, 100)))
+    captured = form(ins, outs, on_device=True)
+    most = 64 * 2200
+    x, y = states(most, 2), list(np.empty((2, most)))
+    want = results(*x)
+    for n in range(most, 0, -64):
+        y[0][:n] = y[1][:n] = 0
+        form([a[:n] for a in x], [a[:n] for a in y])
+        assert np.array_equal(y[0][:n], want[0][:n]) and np.array_equal(y[1][:n], want[1][:n]), n
+    ins[0][:] += 1
+    lib.form_replay(form.form, captured)
+    assert np.array_equal(outs, results(*ins))
