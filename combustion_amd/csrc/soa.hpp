@@ -31,6 +31,10 @@ class SoAForm : public Form {
       return;
     }
     if (!on_device) {
+      // Work queued on the default stream (and, through it, on the streams that synchronize with it) and on the caller's
+      // may still write the inputs or read the outputs, and the host copies begin at once.
+      device::check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+      if (stream) device::check(hipStreamSynchronize(stream), "hipStreamSynchronize");
       // A form with work memory of its own reports on whole calls (the surrogate's fallback count), so its states go in
       // one slice; the others in slices that stay within the staging.
       if (!host_) host_ = std::make_unique<HostArrays>(n_in_, n_out_);

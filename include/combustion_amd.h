@@ -157,9 +157,10 @@ int cb_hip_assemble(const cb_program* p, int32_t form, uint32_t block_size, cb_m
 /* Compiles a form into the code-object cache without touching a GPU. */
 int cb_hip_compile(const cb_program* p, int32_t form, uint32_t block_size);
 /* device.rs:59 call: inputs[n_inputs] and outputs[n_outputs] are SoA arrays of n_states doubles, host or
- * device memory (pointers_are_device). stream is a hipStream_t or NULL. With host pointers the call blocks;
- * with device pointers it is asynchronous unless kernel_ms is requested (then it waits and reports the
- * kernel time measured with HIP events on that stream). */
+ * device memory (pointers_are_device). stream is a hipStream_t or NULL. With host pointers the call waits for the
+ * work queued on `stream` and on the default stream, runs on streams of its own (a module with work memory, the
+ * surrogate, on `stream`) and is complete on return; with device pointers it is asynchronous on `stream` unless
+ * kernel_ms is requested. kernel_ms is the kernels' time measured with HIP events; a call that reports it waits. */
 int cb_hip_call(cb_module* mod, const double* const* inputs, int32_t n_inputs, size_t n_states, double* const* outputs, int32_t n_outputs,
                 int32_t pointers_are_device, void* stream, float* kernel_ms);
 /* Allocation-free variant of cb_hip_call. No counterpart in the reference: it is for callers that cannot allocate

@@ -64,3 +64,16 @@ def test_host_calls_leave_the_tables_of_captured_launches(lib):
     ins[0][:] += 1
     lib.form_replay(form.form, captured)
     assert np.array_equal(outs, results(*ins))
+
+
+@pytest.mark.parametrize("stream,queued", [(8, 8), (None, None), (8, None)], ids=["caller's", "default", "default-before-caller's"])
+def test_host_calls_follow_the_work_queued_before_them(stream, queued, lib):
+    """Copies queued on the caller's or on the default stream, into the inputs and out of the outputs, come first."""
+    form = Form(lib)
+    old, ins = states(100, 3), list(np.zeros((2, 100)))
+    outs, first = list(np.full((2, 100), 5.0)), np.zeros(100)
+    for to, source in ((ins[0], old[0]), (ins[1], old[1]), (first, outs[0])):
+        lib.queue_copy(queued, to.ctypes.data, source.ctypes.data, to.nbytes)
+    form(ins, outs, stream=stream)
+    assert np.array_equal(outs, results(*old))
+    assert np.array_equal(first, np.full(100, 5.0))
