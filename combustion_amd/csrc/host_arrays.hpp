@@ -91,11 +91,14 @@ class HostArrays {
   HostArrays& operator=(const HostArrays&) = delete;
 
   // Whether the arrays may go slice by slice: not where an output overlaps an input at another offset, whose later
-  // states it would overwrite before they are read.
+  // states it would overwrite before they are read, or another output, where the later one of the two has to end on top.
   bool sliceable(const double* const* inputs, size_t n, double* const* outputs) const {
-    for (int o = 0; o < n_out_; o++)
+    for (int o = 0; o < n_out_; o++) {
       for (int i = 0; i < n_in_; i++)
         if (outputs[o] != inputs[i] && outputs[o] < inputs[i] + n && inputs[i] < outputs[o] + n) return false;
+      for (int p = 0; p < o; p++)
+        if (outputs[o] < outputs[p] + n && outputs[p] < outputs[o] + n) return false;
+    }
     return true;
   }
 

@@ -77,3 +77,16 @@ def test_host_calls_follow_the_work_queued_before_them(stream, queued, lib):
     form(ins, outs, stream=stream)
     assert np.array_equal(outs, results(*old))
     assert np.array_equal(first, np.full(100, 5.0))
+
+
+@pytest.mark.parametrize("offset", [0, 1, SLOT // 2])
+@pytest.mark.parametrize("first", ["low", "high"])
+def test_outputs_that_overlap_end_as_the_later_one(first, offset, lib):
+    n = 3 * SLOT // 2  # two slices, and helpers that copy
+    form, ins = Form(lib), states(n)
+    got, want = np.zeros(n + offset), np.zeros(n + offset)
+    views = lambda a: [a[:n], a[offset:]] if first == "low" else [a[offset:], a[:n]]
+    for y, r in zip(views(want), results(*ins)):
+        y[:] = r
+    form(ins, views(got))
+    assert np.array_equal(got, want)
