@@ -4,6 +4,7 @@
 #include <cstring>
 #include <map>
 #include <memory>
+#include <mutex>
 #include <vector>
 
 #include "device.hpp"
@@ -31,6 +32,7 @@ class SoAForm : public Form {
       return;
     }
     if (!on_device) {
+      std::lock_guard<std::mutex> lock(host_mutex_);  // the staging is one for all the threads that share the module
       // Work queued on the default stream (and, through it, on the streams that synchronize with it) and on the caller's
       // may still write the inputs or read the outputs, and the host copies begin at once.
       device::check(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
@@ -105,6 +107,7 @@ class SoAForm : public Form {
   hipEvent_t start_ = nullptr, stop_ = nullptr, done_ = nullptr;
   hipStream_t last_stream_ = nullptr;
   std::unique_ptr<HostArrays> host_;
+  std::mutex host_mutex_;
 
   // The null stream is never captured, and asking costs a runtime call.
   static bool capturing(hipStream_t stream) {

@@ -54,10 +54,15 @@ struct HostForm : combustion::SoAForm {
     size_t n;
   };
   std::vector<Captured> launches;
+  std::mutex mutex;
   HostForm() : SoAForm(2, 2) {}
   void launch(const double* const* in, double* const* out, size_t n, const combustion::Launch&) override {
-    launches.push_back({in, out, n});
-    kernel(launches.back());
+    const Captured c{in, out, n};
+    {
+      std::lock_guard<std::mutex> lock(mutex);
+      launches.push_back(c);
+    }
+    kernel(c);
   }
   static void kernel(const Captured& c) {
     for (size_t s = 0; s < c.n; s++) {

@@ -1,5 +1,6 @@
 """Calls on host arrays (csrc/host_arrays.hpp) and the pointer tables of csrc/soa.hpp, run on the CPU: host_calls.cpp puts
 the plumbing over HIP functions on host memory."""
+import concurrent.futures
 import ctypes as C
 import os
 import subprocess
@@ -90,3 +91,19 @@ def test_outputs_that_overlap_end_as_the_later_one(first, offset, lib):
         y[:] = r
     form(ins, views(got))
     assert np.array_equal(got, want)
+
+
+def test_threads_take_turns_with_the_staging(lib):
+    """Host calls of several threads on one module."""
+    form = Form(lib)
+
+    def calls(seed):
+        for n in (3 * SLOT // 2, 1000, SLOT):
+            ins, outs = states(n, seed), list(np.empty((2, n)))
+            form(ins, outs)
+            if not np.array_equal(outs, results(*ins)):
+                return n
+        return 0
+
+    with concurrent.futures.ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(calls, range(8))) == [0] * 8
