@@ -380,14 +380,16 @@ _addresses = None
 
 
 def _tensor_addresses():
-    """The native helper that reads a list of tensors' addresses (csrc/tensors.cpp); loaded once torch tensors are used."""
+    """The native helper that reads a list of tensors' addresses (csrc/tensors.cpp), loaded once torch tensors are used;
+    without it (a library built where torch was absent) every tensor is examined by itself."""
     global _addresses
     if _addresses is None:
         try:
             import torch  # noqa: F401 (the helper links against it)
             from ._tensors import addresses
-        except ImportError as e:
-            raise ImportError(f"the tensor helper is missing: build it with `python -m combustion_amd.build` ({e})") from e
+        except ModuleNotFoundError:
+            def addresses(sequence, address, length):
+                return -1
         _addresses = addresses
     return _addresses
 

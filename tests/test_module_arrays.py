@@ -1,4 +1,6 @@
 """The arrays that a module's call takes (native.Module.__call__): outputs with room for every state only."""
+import sys
+
 import numpy as np
 import pytest
 
@@ -40,7 +42,7 @@ def module(monkeypatch):
             return 0
 
     monkeypatch.setattr(native, "lib", lambda: Library)
-    monkeypatch.setattr(native, "_tensor_addresses", lambda: lambda *a: -1)  # every array is examined by itself
+    monkeypatch.setattr(native, "_addresses", lambda *a: -1)  # every array is examined by itself
     return mod
 
 
@@ -56,6 +58,15 @@ def test_outputs_have_room_for_every_state(array, module):
     assert module.calls == [8, 8, 8]
     module([array(0), array(0)], [array(0), array(0)])
     assert module.calls[-1] == 0
+
+
+def test_tensors_without_the_native_helper(module, monkeypatch):
+    """A library built where torch was absent has no helper; it serves tensors one by one."""
+    monkeypatch.setattr(native, "_addresses", None)
+    monkeypatch.setitem(sys.modules, "combustion_amd._tensors", None)
+    for n in (5, 6):
+        module([DeviceArray(n), DeviceArray(n)], [DeviceArray(n), DeviceArray(n)])
+    assert module.calls == [5, 6]
 
 
 @pytest.mark.gpu
