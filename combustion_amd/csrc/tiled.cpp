@@ -644,7 +644,7 @@ class RatesMixed {
 // The rates section up to 64 species (with FP32 cores for exp and ln when fast); writes ω to out[0..Ka).
 class RatesStraight {
  public:
-  RatesStraight(const ProgramView& p, bool fast) : t_(rates_text(p, fast)) {
+  explicit RatesStraight(RatesText t) : t_(std::move(t)) {
     kernel_.load(device::compile(t_.source, t_.name, hip_options(true)), t_.name);
     if (t_.split.parts) {
       d_rcp_W_ = upload(t_.split.rcp_W);
@@ -666,7 +666,6 @@ class RatesStraight {
                                         t_.split.parts ? teams : straight, nullptr),
                   "launch rates");
   }
-  const RatesText& text() const { return t_; }
   double *const& rcp_W() const { return d_rcp_W_; }
   double *const& gibbs() const { return d_gibbs_; }
 
@@ -723,7 +722,7 @@ TransportText transport_text(const ProgramView& p, bool f64) {
 
 class TransportStraight {
  public:
-  TransportStraight(const ProgramView& p, bool f64) : t_(transport_text(p, f64)), rcp_T0_(1. / p.chemistry->scales.T0) {
+  TransportStraight(TransportText t, double T0) : t_(std::move(t)), rcp_T0_(1. / T0) {
     kernel_.load(device::compile(t_.source, t_.name, hip_options(true)), t_.name);
     if (split()) {
       d_rcp_W_ = upload(t_.split.rcp_W);
@@ -746,7 +745,6 @@ class TransportStraight {
                   "launch transport");
   }
   bool split() const { return !t_.split.W.empty(); }
-  const TransportText& text() const { return t_; }
 
  private:
   friend class RatesAndTransport;
@@ -792,11 +790,28 @@ std::string rates_and_transport_text(const ProgramView& p, const RatesText& r, c
   return s.str();
 }
 
-// The FP64 kernels that one launch may run both of: teams of four waves in both sections (32 to 53 species: two teams'
-// LDS is 160 KB there), or one lane per state in both.
-bool one_launch(const RatesText& r, const TransportText& t) {
-  const bool split = !t.split.W.empty();
-  return r.split.parts == 4 ? split : r.split.parts == 0 && !split;
+// The FP64 kernels of both sections up to 64 species, and the kernel that runs them in one launch: beside them for teams of
+// four waves in both sections (32 to 53 species: two teams' LDS is 160 KB there), in their place for one lane per state in
+// both, none for other pairs.
+struct BothSections {
+  RatesText rates;
+  TransportText transport;
+  std::string one_launch;
+  bool separate = true;  // the sections' own kernels are launched too
+};
+
+// Whether a form has these kernels: FP64, both sections, neither of them the large mechanisms'.
+bool both_sections(const ProgramView& p, int form_flags) {
+  return (form_flags & kFormBase) == 1 && p.chemistry->options.rates && p.chemistry->options.transport && !tiled_rates(p, form_flags) &&
+         straight_transport(p, form_flags);
+}
+
+BothSections both_sections_text(const ProgramView& p) {
+  BothSections b{rates_text(p, false), transport_text(p, true)};
+  const bool split = !b.transport.split.W.empty();
+  b.separate = split || b.rates.split.parts != 0;
+  if (b.rates.split.parts == 4 ? split : !b.separate) b.one_launch = rates_and_transport_text(p, b.rates, b.transport);
+  return b;
 }
 
 // Both sections of a small batch in one kernel: their blocks run beside each other, where two launches on one stream run
@@ -809,24 +824,24 @@ bool one_launch(const RatesText& r, const TransportText& t) {
 class RatesAndTransport {
  public:
   static constexpr size_t kTeamStates = 64 * 128;
-  RatesAndTransport(const ProgramView& p, const RatesStraight& r, const TransportStraight& t) : r_(r), t_(t), teams_(r.text().split.parts != 0) {
-    kernel_.load(device::compile(rates_and_transport_text(p, r.text(), t.text()), "rates_and_transport", hip_options(true)),
-                 "rates_and_transport");
+  // r and t: the team kernels, whose tables it shares (null for one lane per state, which has none)
+  RatesAndTransport(std::string source, const RatesStraight* r, const TransportStraight* t) : r_(r), t_(t) {
+    kernel_.load(device::compile(source, "rates_and_transport", hip_options(true)), "rates_and_transport");
   }
-  bool takes(size_t n) const { return !teams_ || n <= kTeamStates; }
+  bool takes(size_t n) const { return !r_ || n <= kTeamStates; }
   void launch(const double* const* in, double* const* out, double* const* tout, size_t n, hipStream_t stream) {
     unsigned n32 = (unsigned)n, groups = (unsigned)((n + 63) / 64);
     double pos = 6981463048192., neg = (double)cbrtf(3.40282347e38f);  // reaction.rs:244-256
-    double *rcp_W = r_.rcp_W(), *gibbs = r_.gibbs(), *W = t_.d_W_, *c = t_.d_c_, *v = t_.d_v_, rcp_T0 = t_.rcp_T0_;
+    double *rcp_W = nullptr, *gibbs = nullptr, *W = nullptr, *c = nullptr, *v = nullptr, rcp_T0 = 0;
+    if (r_) rcp_W = r_->rcp_W(), gibbs = r_->gibbs(), W = t_->d_W_, c = t_->d_c_, v = t_->d_v_, rcp_T0 = t_->rcp_T0_;
     void* args[] = {&in, &out, &tout, &n32, &groups, &rcp_W, &gibbs, &pos, &neg, &W, &c, &v, &rcp_T0};
-    device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, teams_ ? 256 : 64, 1, 1, 0, stream, args, nullptr),
+    device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, r_ ? 256 : 64, 1, 1, 0, stream, args, nullptr),
                   "launch rates_and_transport");
   }
 
  private:
-  const RatesStraight& r_;
-  const TransportStraight& t_;
-  bool teams_;
+  const RatesStraight* r_;
+  const TransportStraight* t_;
   device::Kernel kernel_;
 };
 
@@ -875,26 +890,34 @@ class Tiled : public SoAForm {
     const int form = form_flags & kFormBase;
     const bool f64 = form == 1;
     species_ = p.mechanism->species.len();
+    const double T0 = p.chemistry->scales.T0;
+    if (o.rates) n_rates_ = (int)p.mechanism->active;
+    if (both_sections(p, form_flags)) {
+      BothSections b = both_sections_text(p);
+      if (b.separate) {
+        fp64_ = std::make_unique<RatesStraight>(std::move(b.rates));
+        straight_ = std::make_unique<TransportStraight>(std::move(b.transport), T0);
+      }
+      if (!b.one_launch.empty()) small_ = std::make_unique<RatesAndTransport>(std::move(b.one_launch), fp64_.get(), straight_.get());
+      return;
+    }
     if (o.rates) {
-      n_rates_ = (int)p.mechanism->active;
       if (form == 2)
         mixed_ = std::make_unique<RatesMixed>(*p.mechanism);
       else if (tiled_rates(p, form_flags))
         tiled_rates_ = std::make_unique<RatesTiled>(*p.mechanism);
       else
-        fp64_ = std::make_unique<RatesStraight>(p, form == 3);
+        fp64_ = std::make_unique<RatesStraight>(rates_text(p, form == 3));
     }
     if (o.transport) {
       TransportPairs pairs = pairs_of(p, form_flags);
       if (!pairs.source.empty())
-        pairs_ = std::make_unique<TransportPairsKernel>(std::move(pairs), p.chemistry->scales.T0);
+        pairs_ = std::make_unique<TransportPairsKernel>(std::move(pairs), T0);
       else if (straight_transport(p, form_flags))
-        straight_ = std::make_unique<TransportStraight>(p, f64);
+        straight_ = std::make_unique<TransportStraight>(transport_text(p, f64), T0);
       else
         transport_ = std::make_unique<TransportTiled>(p, f64);
     }
-    if (f64 && fp64_ && straight_ && one_launch(fp64_->text(), straight_->text()))
-      small_ = std::make_unique<RatesAndTransport>(p, *fp64_, *straight_);
   }
 
   ~Tiled() override {
@@ -1001,7 +1024,7 @@ class Surrogate : public SoAForm {
       if (w.rates_form == 2)
         mixed_ = std::make_unique<RatesMixed>(m);
       else
-        rates_ = std::make_unique<RatesStraight>(p, true);
+        rates_ = std::make_unique<RatesStraight>(rates_text(p, true));
     }
     // The fallback for states outside the network's box: the plain FP64 transport kernel (the tiled one, which
     // evaluates a list of states in place).
@@ -1169,8 +1192,17 @@ class Surrogate : public SoAForm {
 
 bool tiled_applies(const ProgramView& p) { return p.kind == ProgramKind::Chemistry && !p.chemistry->options.rhs; }
 
+// The texts of the kernels that the form launches. Both sections in one launch: beside the sections' own kernels after the
+// rates, in their place as a whole, marked at the kernel.
 std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
   check_program(p);
+  const std::string mark = "\n// ---- transport ----\n";
+  if (both_sections(p, form_flags)) {
+    BothSections b = both_sections_text(p);
+    if (b.separate) return b.rates.source + (b.one_launch.empty() ? "" : "\n// ---- both in one launch ----\n" + b.one_launch) + mark + b.transport.source;
+    const std::string at = "namespace transport {";
+    return b.one_launch.insert(b.one_launch.find(at), mark);
+  }
   const int form = form_flags & kFormBase;
   const bool mixed = form != 1;
   std::string s;
@@ -1179,7 +1211,7 @@ std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
          : tiled_rates(p, form_flags) ? rates_tiled_text(rates_tiled_tables(*p.mechanism))
                                       : rates_text(p, form == 3).source;
   if (p.chemistry->options.transport) {
-    s += "\n// ---- transport ----\n";
+    s += mark;
     const TransportPairs pairs = pairs_of(p, form_flags);
     if (!pairs.source.empty()) s += pairs.source;
     else if (straight_transport(p, form_flags)) s += transport_text(p, !mixed).source;
@@ -1190,6 +1222,15 @@ std::string tiled_source(const ProgramView& p, int form_flags, unsigned) {
 
 void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
   check_program(p);
+  if (both_sections(p, form_flags)) {
+    const BothSections b = both_sections_text(p);
+    if (b.separate) {
+      device::compile(b.rates.source, b.rates.name, hip_options(true));
+      device::compile(b.transport.source, b.transport.name, hip_options(true));
+    }
+    if (!b.one_launch.empty()) device::compile(b.one_launch, "rates_and_transport", hip_options(true));
+    return;
+  }
   const int form = form_flags & kFormBase;
   const bool mixed = form != 1;
   if (p.chemistry->options.rates) {
@@ -1209,12 +1250,7 @@ void compile_tiled(const ProgramView& p, int form_flags, unsigned) {
     else if (straight_transport(p, form_flags)) {
       const TransportText t = transport_text(p, !mixed);
       device::compile(t.source, t.name, hip_options(true));
-      if (p.chemistry->options.rates && !mixed && !tiled_rates(p, form_flags)) {
-        const RatesText r = rates_text(p, false);
-        if (one_launch(r, t)) device::compile(rates_and_transport_text(p, r, t), "rates_and_transport", hip_options(true));
-      }
-    }
-    else
+    } else
       device::compile(transport_text(transport_tables(*p.mechanism, polynomials(p), p.chemistry->scales.T0), !mixed), "transport_tiled",
                       hip_options(true));
   }
