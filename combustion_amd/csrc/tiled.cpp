@@ -779,14 +779,14 @@ std::string rates_and_transport_text(const ProgramView& p, const RatesText& r, c
        "rates_and_transport(const double* const* __restrict__ in, double* const* __restrict__ out, double* const* __restrict__ tout,\n"
        "                    unsigned n, unsigned groups, const double* __restrict__ rcp_W, const double* __restrict__ gibbs,\n"
        "                    double clamp_pos, double clamp_neg, const double* __restrict__ W, const double* __restrict__ fit_c,\n"
-       "                    const double* __restrict__ fit_v, double rcp_T0) {\n"
+       "                    const double* __restrict__ fit_v, double rcp_T0, unsigned first) {\n"
        "  if (blockIdx.x < groups)\n"
        "    transport::run(blockIdx.x, in, tout, n, "
-    << (teams ? "rcp_W, W, fit_c, fit_v, rcp_T0" : "0u")
+    << (teams ? "rcp_W, W, fit_c, fit_v, rcp_T0" : "first")
     << ");\n"
        "  else\n"
        "    rates::run(blockIdx.x - groups, in, out, n, "
-    << (teams ? "rcp_W, gibbs, clamp_pos, clamp_neg" : "0u") << ");\n}\n";
+    << (teams ? "rcp_W, gibbs, clamp_pos, clamp_neg" : "first") << ");\n}\n";
   return s.str();
 }
 
@@ -830,13 +830,18 @@ class RatesAndTransport {
   }
   bool takes(size_t n) const { return !r_ || n <= kTeamStates; }
   void launch(const double* const* in, double* const* out, double* const* tout, size_t n, hipStream_t stream) {
-    unsigned n32 = (unsigned)n, groups = (unsigned)((n + 63) / 64);
     double pos = 6981463048192., neg = (double)cbrtf(3.40282347e38f);  // reaction.rs:244-256
     double *rcp_W = nullptr, *gibbs = nullptr, *W = nullptr, *c = nullptr, *v = nullptr, rcp_T0 = 0;
     if (r_) rcp_W = r_->rcp_W(), gibbs = r_->gibbs(), W = t_->d_W_, c = t_->d_c_, v = t_->d_v_, rcp_T0 = t_->rcp_T0_;
-    void* args[] = {&in, &out, &tout, &n32, &groups, &rcp_W, &gibbs, &pos, &neg, &W, &c, &v, &rcp_T0};
-    device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, r_ ? 256 : 64, 1, 1, 0, stream, args, nullptr),
-                  "launch rates_and_transport");
+    // two lanes a state: a launch of all states below 2^31 would have up to 2^32 threads, one more than a launch may
+    constexpr size_t most = size_t(1) << 30;
+    for (size_t first = 0; first < n; first += most) {
+      const size_t end = std::min(n, first + most);
+      unsigned from = (unsigned)first, to = (unsigned)end, groups = (unsigned)((end - first + 63) / 64);
+      void* args[] = {&in, &out, &tout, &to, &groups, &rcp_W, &gibbs, &pos, &neg, &W, &c, &v, &rcp_T0, &from};
+      device::check(hipModuleLaunchKernel(kernel_.function, 2 * groups, 1, 1, r_ ? 256 : 64, 1, 1, 0, stream, args, nullptr),
+                    "launch rates_and_transport");
+    }
   }
 
  private:
