@@ -13,8 +13,8 @@
 //      then every part adds the rows of its own species and writes them out
 //
 // Bound: FP64 VALU issue. Per 64 states of the 53-species mechanism it issues 17.3 k VALU instructions where the
-// one-lane kernel issued 23.4 k (no accumulation-register moves, base-2 exponentials without clamps of their own, one
-// exponential per rate constant, one factor per product species) at one wave per SIMD; with two waves per SIMD and the
+// one-lane kernel issued 23.4 k (no accumulation-register moves, exponentials without clamps of their own and with
+// a reduction of one rounding, one exponential per rate constant, one factor per product species) at one wave per SIMD; with two waves per SIMD and the
 // parts' scalar constants and LDS reads beside the other wave's arithmetic, 2^20 states take 0.80 ms against 1.19 ms,
 // and a single wavefront's worth of states 25 against 75 us (a quarter of the reactions per wave). What is left of
 // it: a block of 128 states spends 34 of its 54 k cycles in the reactions (27 k of them issue), 7 k in the Gibbs
@@ -22,10 +22,12 @@
 // to 0.95 ms: 168 registers spill), persistent blocks with the teams on barriers of their own (0.82 to 0.9 ms: the
 // loop's invariants spill), rows of independent instructions pinned by scheduling barriers (0.80 ms, compile times of
 // minutes).
+// Rounding: 3.6e-15 of the state's largest rate on average (4096 states, against the program in 80-bit arithmetic), 4.7e-15
+// for the one-lane kernel and 4.0e-15 with the library's functions.
 // Required defines: NAME, K, KA (active species), PARTS (waves per team, even), TEAMS (teams per block), FAST (1: exp
-// and ln on the FP32 cores, in natural units; 0: FP64 polynomials, exponents and logarithms in base 2).
+// and ln on the FP32 cores; 0: FP64 polynomials).
 // Tables: rcp_W[K], gibbs[KA][15] = the split temperature and the two 7-coefficient pieces of g (low first), in the
-// basis 1, L, T, T², T³, T⁴, 1/T with L = log2 T (FAST: ln T) and in units of 1/log2(e) (FAST: 1).
+// basis 1, ln T, T, T², T³, T⁴, 1/T.
 
 typedef const double __attribute__((address_space(4))) * table;  // read by scalar loads at wave-uniform indices
 
@@ -33,7 +35,7 @@ typedef const double __attribute__((address_space(4))) * table;  // read by scal
 #define P0_R (101325.0 / RGAS)
 #define FLT_MIN_D 1.1754943508222875e-38
 #define FLT_MAX_D 3.4028234663852886e38
-#define LOG2_FLT_MAX 0x1.fffffffa3aae2p+6
+#define LN_FLT_MAX 0x1.62e42fefa39efp+6
 #define SCALE 0x1p+100
 #define COLS (64 * TEAMS)
 #define KP ((K + PARTS - 1) / PARTS)
@@ -58,9 +60,11 @@ __device__ __forceinline__ void rcp64_rows(double* x) {
   ROW x[i] = __builtin_fma(r[i], e[i], r[i]);
 }
 
+// exp64_rows: e^x. log_rows and pow_rows: the logarithm to a base of the kernel's own (FAST: e, else 2) and its inverse.
+// log64: ln x.
 #if FAST
-// e^x and ln x with FP32 cores: 2^n 2^f with the FP64 reduction x log2 e = n + f and v_exp_f32; the FP64 exponent and
-// mantissa split and v_log_f32
+// With FP32 cores: 2^n 2^f with the FP64 reduction x log2 e = n + f and v_exp_f32; the FP64 exponent and mantissa split and
+// v_log_f32
 template <int N>
 __device__ __forceinline__ void exp64_rows(double* x) {
   double y[N], n[N];
@@ -74,7 +78,11 @@ __device__ __forceinline__ void exp64_rows(double* x) {
   ROW x[i] = __builtin_ldexp((double)f[i], (int)n[i]);
 }
 template <int N>
-__device__ __forceinline__ void log64_rows(double* x) {
+__device__ __forceinline__ void pow_rows(double* x) {
+  exp64_rows<N>(x);
+}
+template <int N>
+__device__ __forceinline__ void log_rows(double* x) {
   ROW {
     const long long b = __double_as_longlong(x[i]);
     const int e = (int)((b >> 52) & 0x7FF) - 1023;
@@ -82,16 +90,17 @@ __device__ __forceinline__ void log64_rows(double* x) {
     x[i] = ((double)e + (double)__builtin_amdgcn_logf((float)m)) * 0.6931471805599453;
   }
 }
+__device__ __forceinline__ double log64(double x) {
+  log_rows<1>(&x);
+  return x;
+}
 #else
-// 2^y for |y| < 2^31: n = rint(y) from the low word of y + 1.5·2^52, r = y - n exactly, the Chebyshev interpolant of
-// 2^r of degree 10 on |r| <= 1/2 (exp_coefficients.py; relative error below 5e-16) and v_ldexp_f64, which gives 0 and
-// +inf outside the FP64 range: 14 instructions. Base 2 because its reduction needs no rounded ln 2.
+// 2^(t + r) with t an integer plus 1.5·2^52, of which the low word is read, and |r| <= 1/2: the Chebyshev interpolant of 2^r
+// of degree 10 (exp_coefficients.py; relative error below 5e-16) and v_ldexp_f64, which gives 0 and +inf outside the FP64
+// range
 template <int N>
-__device__ __forceinline__ void exp64_rows(double* y) {
-  double t[N], r[N], p[N];
-  ROW t[i] = y[i] + 0x1.8p+52;
-  ROW r[i] = t[i] - 0x1.8p+52;
-  ROW r[i] = y[i] - r[i];
+__device__ __forceinline__ void pow2_rows(double* y, const double* t, const double* r) {
+  double p[N];
   ROW p[i] = __builtin_fma(0x1.e6063f7217bc6p-28, r[i], 0x1.b675bca4eeebbp-24);
   const double c[9] = {0x1.62bfd47773353p-20, 0x1.ffcb54062e698p-17, 0x1.430913096fd9fp-13, 0x1.5d87fe9d7a584p-10, 0x1.3b2ab6fba1ddap-7,
                        0x1.c6b08d703ce49p-5,  0x1.ebfbdff82c598p-3,  0x1.62e42fefa3a19p-1,  1.0};
@@ -101,25 +110,44 @@ __device__ __forceinline__ void exp64_rows(double* y) {
   }
   ROW y[i] = __builtin_ldexp(p[i], (int)(unsigned)__double_as_longlong(t[i]));
 }
-// log2 x for x > 0: x = 2^e m with m in [sqrt(1/2), sqrt(2)), log2 m = s P(s²) with s = (m-1)/(m+1) (the atanh
-// series; P the Chebyshev interpolant of degree 7, relative error 1.4e-17)
+// For |y| < 2^31: n = rint(y), r = y - n exactly: 14 instructions.
 template <int N>
-__device__ __forceinline__ void log64_rows(double* x) {
-  double num[N], den[N], r[N], z[N], p[N];
-  int e[N];
+__device__ __forceinline__ void pow_rows(double* y) {
+  double t[N], r[N];
+  ROW t[i] = y[i] + 0x1.8p+52;
+  ROW r[i] = t[i] - 0x1.8p+52;
+  ROW r[i] = y[i] - r[i];
+  pow2_rows<N>(y, t, r);
+}
+// For |x| < 2^30: n = rint(x log2 e), r = x log2 e - n in one rounding: 14 instructions too. The FP64 log2 e is off by 1.4e-17
+// of itself, an eighth of the rounding that x comes with; scaling the exponents' coefficients by it beforehand costs a
+// rounding of every coefficient (mean error of the rates 4.4e-15 instead of 3.6e-15).
+template <int N>
+__device__ __forceinline__ void exp64_rows(double* x) {
+  double t[N], r[N];
+  ROW t[i] = __builtin_fma(x[i], 0x1.71547652b82fep+0, 0x1.8p+52);
+  ROW r[i] = t[i] - 0x1.8p+52;
+  ROW r[i] = __builtin_fma(x[i], 0x1.71547652b82fep+0, -r[i]);
+  pow2_rows<N>(x, t, r);
+}
+// log2 m for x = 2^e m > 0 with m in [sqrt(1/2), sqrt(2)): s P(s²) with s = (m-1)/(m+1) (the atanh series; P the
+// Chebyshev interpolant of degree 7, exp_coefficients.py, relative error 1.4e-17)
+template <int N>
+__device__ __forceinline__ void mantissa_log_rows(const double* x, double* e, double* s, double* p) {
+  double num[N], den[N], r[N], z[N];
   ROW {
     const double m = __builtin_amdgcn_frexp_mant(x[i]);
     const int low = m < 0x1.6a09e667f3bcdp-1;
-    e[i] = __builtin_amdgcn_frexp_exp(x[i]) - low;
+    e[i] = (double)(__builtin_amdgcn_frexp_exp(x[i]) - low);
     num[i] = __builtin_ldexp(m, low);
     den[i] = r[i] = num[i] + 1.0;
     num[i] -= 1.0;
   }
   rcp64_rows<N>(r);
-  ROW x[i] = num[i] * r[i];
-  ROW z[i] = __builtin_fma(-x[i], den[i], num[i]);
-  ROW x[i] = __builtin_fma(z[i], r[i], x[i]);
-  ROW z[i] = x[i] * x[i];
+  ROW s[i] = num[i] * r[i];
+  ROW z[i] = __builtin_fma(-s[i], den[i], num[i]);
+  ROW s[i] = __builtin_fma(z[i], r[i], s[i]);
+  ROW z[i] = s[i] * s[i];
   ROW p[i] = __builtin_fma(0x1.b592d3c48c41cp-3, z[i], 0x1.c46e1440404d7p-3);
   const double c[6] = {0x1.0ca160627dbfcp-2, 0x1.484afb7a67652p-2, 0x1.a61762d693934p-2,
                        0x1.2776c50ee39dcp-1, 0x1.ec709dc3a047dp-1, 0x1.71547652b82fep+1};
@@ -127,15 +155,22 @@ __device__ __forceinline__ void log64_rows(double* x) {
   for (int j = 0; j < 6; j++) {
     ROW p[i] = __builtin_fma(p[i], z[i], c[j]);
   }
-  ROW x[i] = __builtin_fma(x[i], p[i], (double)e[i]);
+}
+template <int N>
+__device__ __forceinline__ void log_rows(double* x) {
+  double e[N], s[N], p[N];
+  mantissa_log_rows<N>(x, e, s, p);
+  ROW x[i] = __builtin_fma(s[i], p[i], e[i]);
+}
+// (one rounding at the size of the result: with ln 2 times log2 x the rates' mean error was 4.0e-15 instead of 3.6e-15)
+__device__ __forceinline__ double log64(double x) {
+  double e, s, p;
+  mantissa_log_rows<1>(&x, &e, &s, &p);
+  return __builtin_fma(e, 0x1.62e42fefa39efp-1, s * p * 0x1.62e42fefa39efp-1);
 }
 #endif
 __device__ __forceinline__ double exp64(double x) {
   exp64_rows<1>(&x);
-  return x;
-}
-__device__ __forceinline__ double log64(double x) {
-  log64_rows<1>(&x);
   return x;
 }
 
@@ -172,7 +207,9 @@ NAME(const double* const* __restrict__ in, double* const* __restrict__ out, unsi
   }
   lds_v[part * COLS + col] = sum;
   lds_v[(PARTS + part) * COLS + col] = positive;
-  const double rcpT = rcp64(T), L = log64(T), T2 = T * T, T3 = T * T2, T4 = T2 * T2;
+  // a second Newton step: 1/T stands in every exponent, tens of times over
+  const double rT1 = rcp64(T), rcpT = __builtin_fma(rT1, __builtin_fma(-T, rT1, 1.0), rT1);
+  const double L = log64(T), T2 = T * T, T3 = T * T2, T4 = T2 * T2;
   const double C_tot = P * (1.0 / RGAS) * rcpT;
   __syncthreads();
   sum = lds_v[col];
@@ -222,15 +259,15 @@ NAME(const double* const* __restrict__ in, double* const* __restrict__ out, unsi
 #define F(k) f_[(k) * COLS]
 #define EN(k) e_[(k) * COLS]
   const double C0 = SCALE * P0_R * rcpT, rcpC0 = T * (1.0 / (SCALE * P0_R));
-#if FAST
   const double rcpT2 = rcpT * rcpT;
-#define KF(x) exp64(x)
 #define LIMIT(x) __builtin_fmin(FLT_MAX_D, x)
+#if FAST
+#define KF(x) exp64(x)
 #else
-  // 1/T and log2 T as the rate constants' exponents take them, kept where 2^31 bounds the exponents (below 1 mK and
+  // 1/T and ln T as the rate constants' exponents take them, kept where 2^30 bounds the exponents (below 1 mK and
   // outside the FP64 range every rate constant is 0 or FLT_MAX by then)
-  const double rT = __builtin_fmin(rcpT, 1e3), LT = __builtin_fmin(__builtin_fmax(L, -1100.0), 1100.0);
-#define KF(x) exp64(__builtin_fmin(LOG2_FLT_MAX, x))
+  const double rT = __builtin_fmin(rcpT, 1e3), LT = __builtin_fmin(__builtin_fmax(L, -760.0), 760.0);
+#define KF(x) exp64(__builtin_fmin(LN_FLT_MAX, x))
 #endif
 @SECTIONS@
   // 3. sums over the parts

@@ -18,11 +18,11 @@ namespace combustion {
 namespace {
 
 constexpr double kLog2e = 1.4426950408889634;
+// A compiler-only fence between segments: each reads the LDS values it uses instead of keeping an earlier read live.
+const char* const kFence = "  asm volatile(\"\" ::: \"memory\");\n";
 // Reactions per segment. A segment's LDS values are read while the segment before it computes, and its reactions are
 // evaluated side by side, factor by factor. One and two reactions at a time took 0.84 and 0.81 ms per 2^20 states of
 // the 53-species mechanism, four 0.80 ms at 245 of the 256 registers.
-// A compiler-only fence between segments: each reads the LDS values it uses instead of keeping an earlier read live.
-const char* const kFence = "  asm volatile(\"\" ::: \"memory\");\n";
 constexpr size_t kSegment = 4, kThirdBodySegment = 2;
 
 std::string literal(double x) {
@@ -31,22 +31,21 @@ std::string literal(double x) {
   return buf;
 }
 
-// Text of one mechanism's reactions. Exponents and logarithms are in units of `u`: log2(e) with FP64 polynomials in
-// base 2, 1 with FP32 cores in natural units.
+// Text of one mechanism's reactions. Falloff's logarithms, and the power taken of them again, are to the base that the
+// kernel's log_rows and pow_rows have: 2 with the FP64 polynomials, e with the FP32 cores.
 class Writer {
  public:
-  Writer(const Mechanism& m, bool fast) : m_(m), fast_(fast), u_(fast ? 1. : kLog2e) {}
+  Writer(const Mechanism& m, bool fast) : m_(m), fast_(fast), falloff_unit_(fast ? 1. : kLog2e) {}
 
-  // min(FLT_MAX, A T^β e^(-θ/T)) (reaction.rs:113-139) as (β·L + a/T) + ln A under one exponential; with the FP32
-  // cores the power of T nearest β stays outside it, which keeps the FP32 argument's rounding where the reference's
-  // form puts it.
+  // min(FLT_MAX, A T^β e^(-θ/T)) (reaction.rs:113-139) as (β·L + a/T) + ln A under one exponential, the power of T
+  // nearest β outside it: the exponent's rounding error grows with its terms (with T^β in the exponent whole the rates'
+  // mean error against 80 bits was 3.76e-15 of the state's largest, as it is 3.64e-15).
   struct Rate {
     double beta, a, lnA, A;
     const char* factor;  // outside the exponential, or null
     bool constant() const { return beta == 0. && a == 0.; }
   };
   Rate rate(const RateConstant& k) const {
-    if (!fast_) return {k.temperature_exponent, -k.activation_temperature * u_, std::log2(k.preexponential_factor), k.preexponential_factor, nullptr};
     const double beta = k.temperature_exponent;
     struct { double above, shift; const char* factor; } const up[] = {{3.5, 4., "T4"}, {2.5, 3., "T3"}, {1.5, 2., "T2"}, {0.5, 1., "T"}};
     const char* factor = nullptr;
@@ -64,7 +63,8 @@ class Writer {
   const char* log_T() const { return fast_ ? "L" : "LT"; }
   const char* rcp_T() const { return fast_ ? "rcpT" : "rT"; }
   std::string limited(const Rate& r, const std::string& e) const {
-    if (!fast_) return r.constant() ? literal(std::min((double)FLT_MAX, r.A)) : e;
+    // without a factor the FP64 exponent is bounded instead (see evaluate)
+    if (!fast_ && !r.factor) return r.constant() ? literal(std::min((double)FLT_MAX, r.A)) : e;
     const std::string v = r.constant() ? literal(r.A) : e;
     return std::string("LIMIT(") + (r.factor ? std::string(r.factor) + " * " : "") + v + ")";
   }
@@ -72,7 +72,7 @@ class Writer {
   std::string rate_constant(const RateConstant& k) const {
     const Rate r = rate(k);
     const std::string x = sum_terms(r.beta, log_T(), r.a, rcp_T());
-    return limited(r, r.constant() ? "" : "KF(" + x + " + " + literal(r.lnA) + ")");
+    return limited(r, r.constant() ? "" : (r.factor ? "exp64(" : "KF(") + x + " + " + literal(r.lnA) + ")");
   }
 
   // Exponents of several exponentials, evaluated together (`name`[i]).
@@ -103,7 +103,8 @@ class Writer {
       row([&](const Rate& r, const std::string&) { return " = " + literal(r.a) + " * " + rcp_T(); });
       row([&](const Rate& r, const std::string&) { return " += " + literal(r.beta) + " * " + log_T(); });
       row([&](const Rate& r, const std::string&) { return " += " + literal(r.lnA); });
-      if (!fast_) row([&](const Rate&, const std::string& v) { return " = __builtin_fmin(LOG2_FLT_MAX, " + v + ")"; });
+      for (size_t i = 0; i < nr && !fast_; i++)
+        if (!x.rates[i].factor) s << "    " << name << "[" << i << "] = __builtin_fmin(LN_FLT_MAX, " << name << "[" << i << "]);\n";
     }
     for (size_t i = 0; i < x.others.size(); i++)
       s << "    " << name << "[" << nr + i << "] = " << bounded(x.others[i]) << ";\n";
@@ -137,12 +138,12 @@ class Writer {
       const auto& ks = levels[i].second;
       s << "    const double l" << i << " = ";
       if (ks.size() == 1 && ks[0].preexponential_factor > 0) {
-        const std::string x = sum_terms(ks[0].temperature_exponent, L, -ks[0].activation_temperature * u_, rT);
-        s << literal(std::log(ks[0].preexponential_factor) * u_) << (x.empty() ? "" : " + ") << x;
+        const std::string x = sum_terms(ks[0].temperature_exponent, L, -ks[0].activation_temperature, rT);
+        s << literal(std::log(ks[0].preexponential_factor)) << (x.empty() ? "" : " + ") << x;
       } else {
         s << "log64(";
         for (size_t j = 0; j < ks.size(); j++) {
-          const std::string x = sum_terms(ks[j].temperature_exponent, L, -ks[j].activation_temperature * u_, rT);
+          const std::string x = sum_terms(ks[j].temperature_exponent, L, -ks[j].activation_temperature, rT);
           s << (j ? " + " : "") << literal(ks[j].preexponential_factor) << " * exp64(" << (x.empty() ? "0.0" : x) << ")";
         }
         s << ")";
@@ -151,12 +152,12 @@ class Writer {
     }
     s << "    double lk = l" << levels.size() - 1 << ";\n";
     if (levels.size() > 1) {
-      s << "    const double lP = log64(C_tot) + L + " << literal(std::log(R) * u_) << ";\n";
+      s << "    const double lP = log64(C_tot) + L + " << literal(std::log(R)) << ";\n";
       for (int i = (int)levels.size() - 2; i >= -1; i--) {
-        const double edge = std::log(levels[i + 1].first) * u_;
+        const double edge = std::log(levels[i + 1].first);
         s << "    if (lP <= " << literal(edge) << ") lk = ";
         if (i >= 0) {
-          const double lo = std::log(levels[i].first) * u_;
+          const double lo = std::log(levels[i].first);
           s << "l" << i << " + (l" << i + 1 << " - l" << i << ") * ((lP - " << literal(lo) << ") * " << literal(1. / (edge - lo)) << ");\n";
         } else {
           s << "l0;\n";
@@ -230,9 +231,9 @@ class Writer {
       center[i] = {-1, -1, -1};
       if (rs[i]->model != ReactionModel::Troe) continue;
       const Troe& t = rs[i]->troe;
-      center[i][0] = (int)x.add("T * " + literal(-u_ / t.T3));
-      if (t.T1 < 1e30) center[i][1] = (int)x.add("T * " + literal(-u_ / t.T1));
-      if (std::isfinite(t.T2)) center[i][2] = (int)x.add("rcpT * " + literal(-t.T2 * u_));
+      center[i][0] = (int)x.add("T * " + literal(-1. / t.T3));
+      if (t.T1 < 1e30) center[i][1] = (int)x.add("T * " + literal(-1. / t.T1));
+      if (std::isfinite(t.T2)) center[i][2] = (int)x.add("rcpT * " + literal(-t.T2));
     }
     s << evaluate(x, "x");
     size_t troes = 0;
@@ -248,7 +249,7 @@ class Writer {
     if (troes) {
       // ln Fcent and ln Pr, then F = 10^(log Fcent / (1 + f1²)) with f1 = lp/d, and Pr/(1 + Pr): both quotients from
       // one reciprocal
-      const double ln10 = std::log(10.) * u_;
+      const double ln10 = std::log(10.) * falloff_unit_;
       std::vector<size_t> at;
       for (size_t i = 0; i < n; i++)
         if (rs[i]->model == ReactionModel::Troe) at.push_back(i);
@@ -263,7 +264,7 @@ class Writer {
           << (center[i][1] >= 0 ? " * " + e(center[i][1]) : "") << (center[i][2] >= 0 ? " + " + e(center[i][2]) : "") << ";\n"
           << "    l[" << 2 * j + 1 << "] = Pr" << i << " + FLT_MIN_D;\n";
       }
-      s << "    log64_rows<" << 2 * troes << ">(l);\n    double w[" << troes << "];\n";
+      s << "    log_rows<" << 2 * troes << ">(l);\n    double w[" << troes << "];\n";
       for (size_t j = 0; j < troes; j++) {
         const size_t i = at[j];
         const std::string lF = "l[" + std::to_string(2 * j) + "]", lPr = "l[" + std::to_string(2 * j + 1) + "]";
@@ -278,7 +279,7 @@ class Writer {
         s << "    f[" << j << "] = " << bounded("l[" + std::to_string(2 * j) + "] * (dd" + std::to_string(i) + " * (w[" + std::to_string(j) + "] * qb" +
                                                std::to_string(i) + "))") << ";\n";
       }
-      s << "    exp64_rows<" << troes << ">(f);\n";
+      s << "    pow_rows<" << troes << ">(f);\n";
       for (size_t j = 0; j < troes; j++) {
         const size_t i = at[j];
         s << "    double " << id("k", i) << " = " << literal(rs[i]->rate_constant.preexponential_factor) << " * " << id("high", i) << " * f[" << j
@@ -299,10 +300,10 @@ class Writer {
     const SRI& x = r.sri;
     s << third_body(r, "M") << "    const double kinf = " << rate_constant(r.rate_constant) << ";\n"
       << "    const double Pr = M * " << rate_constant(r.k0) << " * rcp64(kinf + FLT_MIN_D);\n"
-      << "    const double lg = log64(Pr + FLT_MIN_D) * " << literal(1. / (std::log(10.) * u_)) << ";\n"
+      << "    const double lg = log64(Pr + FLT_MIN_D) * " << literal(1. / std::log(10.)) << ";\n"
       << "    const double X = rcp64(1.0 + lg * lg);\n"
-      << "    const double base = " << literal(x.A) << " * exp64(" << bounded("rcpT * " + literal(-x.B * u_)) << ")";
-    if (x.C != 0.) s << " + exp64(" << bounded("T * " + literal(-u_ / x.C)) << ")";
+      << "    const double base = " << literal(x.A) << " * exp64(" << bounded("rcpT * " + literal(-x.B)) << ")";
+    if (x.C != 0.) s << " + exp64(" << bounded("T * " + literal(-1. / x.C)) << ")";
     s << ";\n    double k0 = " << literal(x.D) << " * exp64(" << bounded("X * log64(base)") << ");\n";
     if (x.E != 0.) s << "    k0 *= exp64(" << bounded(literal(x.E) + " * L") << ");\n";
     s << "    k0 *= kinf * Pr * rcp64(Pr + 1.0);\n";
@@ -413,7 +414,7 @@ class Writer {
 
   const Mechanism& m_;
   bool fast_;
-  double u_;
+  double falloff_unit_;
   int number_ = 0;
   mutable std::set<std::pair<char, size_t>> reads_;
 };
@@ -486,14 +487,12 @@ RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast, b
   replace(t.source, "@STORE@\n", store.str());
   replace(t.source, "@ADD@\n", add.str());
   for (size_t k = 0; k < K; k++) t.rcp_W.push_back(1. / m.species.molar_mass[k]);
-  const double u = fast ? 1. : kLog2e;
   for (size_t k = 0; k < KA; k++) {
     const NASA7& n = m.species.thermodynamics[k];
     t.gibbs.push_back(std::isnan(n.temperature_split) ? INFINITY : n.temperature_split);
     for (const auto& a : n.pieces) {
-      // the arrangement of reaction.rs:78; the logarithm's coefficient is the same in either base
-      const double g[7] = {u * (a[0] - a[6]), -a[0], -u * a[1] / 2., u * (1. / 3. - 1. / 2.) * a[2], u * (1. / 4. - 1. / 3.) * a[3],
-                           u * (1. / 5. - 1. / 4.) * a[4], u * a[5]};
+      // the arrangement of reaction.rs:78
+      const double g[7] = {a[0] - a[6], -a[0], -a[1] / 2., (1. / 3. - 1. / 2.) * a[2], (1. / 4. - 1. / 3.) * a[3], (1. / 5. - 1. / 4.) * a[4], a[5]};
       t.gibbs.insert(t.gibbs.end(), g, g + 7);
     }
   }
