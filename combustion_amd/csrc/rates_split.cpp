@@ -430,8 +430,8 @@ void replace(std::string& text, const std::string& what, const std::string& with
 RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast, bool one_team) {
   const size_t K = m.species.len(), KA = m.active;
   RatesSplit t;
-  // Eight waves per CU (two per SIMD, 256 registers each): two teams of four waves where their LDS fits (up to 53
-  // species with one of them inert), since each part pays for the shared prologue and the sums, else one team of eight.
+  // Eight waves per CU (two per SIMD, 256 registers each): two teams of four waves where their LDS fits (up to 54
+  // species with one of them inert, which take all of it), since each part pays for the shared prologue and the sums, else one team of eight.
   t.teams = (2 * KA + K) * 128 * sizeof(double) <= 160 * 1024 ? 2 : 1;
   t.parts = 8 / t.teams;
   if (one_team) t.teams = 1;

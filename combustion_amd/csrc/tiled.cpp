@@ -791,7 +791,7 @@ std::string rates_and_transport_text(const ProgramView& p, const RatesText& r, c
 }
 
 // The FP64 kernels of both sections up to 64 species, and the kernel that runs them in one launch: beside them for teams of
-// four waves in both sections (32 to 53 species: two teams' LDS is 160 KB there), in their place for one lane per state in
+// four waves in both sections (32 to 54 species, one of them inert: two teams' LDS is all 160 KB there), in their place for one lane per state in
 // both, none for other pairs.
 struct BothSections {
   RatesText rates;
