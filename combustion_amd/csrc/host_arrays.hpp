@@ -6,9 +6,9 @@
 #include <algorithm>
 #include <condition_variable>
 #include <cstring>
+#include <exception>
 #include <functional>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -21,8 +21,9 @@ class CopyTeam {
  public:
   explicit CopyTeam(int helpers) {
     try {
+      threads_.reserve(helpers);
       for (int i = 0; i < helpers; i++) threads_.emplace_back([this] { work(); });
-    } catch (const std::system_error&) {  // fewer helpers, or none
+    } catch (const std::exception&) {  // no thread or no memory for one: fewer helpers, or none
     }
   }
   ~CopyTeam() {

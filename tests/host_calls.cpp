@@ -1,9 +1,19 @@
 // A form whose kernel runs on the host (out0 = in0 + in1, out1 = in0 in1), over HIP functions on host memory: the launch
 // plumbing of csrc/soa.hpp and csrc/host_arrays.hpp without a GPU (test_host_calls.py).
+#include <atomic>
 #include <cstdlib>
 #include <map>
+#include <new>
 
 #include "soa.hpp"
+
+static std::atomic<long> allocations_left{-1};  // the allocation after these fails; never where negative
+void* operator new(size_t bytes) {
+  if (allocations_left >= 0 && allocations_left-- == 0) throw std::bad_alloc();
+  return std::malloc(bytes);
+}
+void operator delete(void* p) noexcept { std::free(p); }
+void operator delete(void* p, size_t) noexcept { std::free(p); }
 
 namespace {
 struct Copy {
@@ -15,8 +25,10 @@ std::mutex pending_mutex;
 std::map<hipStream_t, std::vector<Copy>> pending;  // queued on a stream, done when it is waited for
 void drain(hipStream_t s) {
   std::lock_guard<std::mutex> lock(pending_mutex);
-  for (const Copy& c : pending[s]) std::memcpy(c.to, c.from, c.bytes);
-  pending[s].clear();
+  const auto at = pending.find(s);
+  if (at == pending.end()) return;
+  for (const Copy& c : at->second) std::memcpy(c.to, c.from, c.bytes);
+  pending.erase(at);
 }
 }  // namespace
 
@@ -76,9 +88,17 @@ struct HostForm : combustion::SoAForm {
 extern "C" {
 void* form_new() { return new HostForm; }
 void form_free(void* f) { delete (HostForm*)f; }
-void form_call(void* f, const double* const* in, size_t n, double* const* out, int on_device, void* stream) {
-  ((HostForm*)f)->call(in, n, out, on_device != 0, (hipStream_t)stream, nullptr);
+// 0, or 1 where the call failed.
+int form_call(void* f, const double* const* in, size_t n, double* const* out, int on_device, void* stream) {
+  try {
+    ((HostForm*)f)->call(in, n, out, on_device != 0, (hipStream_t)stream, nullptr);
+  } catch (const std::exception&) {
+    return 1;
+  }
+  return 0;
 }
+void fail_allocation(long n) { allocations_left = n; }
+long unused_allocations() { return allocations_left; }
 size_t form_launches(void* f) { return ((HostForm*)f)->launches.size(); }
 // A launch again with the table it was given, as a captured graph replays it.
 void form_replay(void* f, size_t launch) { HostForm::kernel(((HostForm*)f)->launches[launch]); }

@@ -25,6 +25,8 @@ def lib(tmp_path_factory):
     l.form_launches.argtypes = l.form_free.argtypes = [C.c_void_p]
     l.form_replay.argtypes = [C.c_void_p, C.c_size_t]
     l.form_call.argtypes = [C.c_void_p, C.POINTER(C.c_void_p), C.c_size_t, C.POINTER(C.c_void_p), C.c_int, C.c_void_p]
+    l.fail_allocation.argtypes = [C.c_long]
+    l.unused_allocations.restype = C.c_long
     l.queue_copy.argtypes = [C.c_void_p, C.c_void_p, C.c_void_p, C.c_size_t]
     return l
 
@@ -38,7 +40,8 @@ class Form:
 
     def __call__(self, ins, outs, n=None, on_device=False, stream=None):
         table = lambda arrays: (C.c_void_p * 2)(*[a.ctypes.data for a in arrays])
-        self.lib.form_call(self.form, table(ins), len(ins[0]) if n is None else n, table(outs), int(on_device), stream)
+        if self.lib.form_call(self.form, table(ins), len(ins[0]) if n is None else n, table(outs), int(on_device), stream):
+            raise MemoryError
         return self.lib.form_launches(self.form) - 1
 
 
@@ -107,3 +110,29 @@ def test_threads_take_turns_with_the_staging(lib):
 
     with concurrent.futures.ThreadPoolExecutor(4) as pool:
         assert list(pool.map(calls, range(8))) == [0] * 8
+
+
+@pytest.mark.timeout(100)
+def test_a_host_call_that_runs_out_of_memory_fails_by_itself(lib):
+    """Each allocation of a call in turn (the helper threads' among them) fails: the call works without or reports it, and
+    the next one is whole."""
+    ins = states(3 * SLOT // 2)
+    failed = 0
+    for nth in range(1000):
+        form, outs = Form(lib), list(np.zeros((2, len(ins[0]))))
+        lib.fail_allocation(nth)
+        try:
+            form(ins, outs)
+            done = True
+        except MemoryError:
+            done = False
+        finally:
+            unused = lib.unused_allocations() > 0
+            lib.fail_allocation(-1)
+        failed += not done
+        if not done:
+            form(ins, outs)
+        assert np.array_equal(outs, results(*ins)), nth
+        if unused:
+            break
+    assert 0 < failed < nth
