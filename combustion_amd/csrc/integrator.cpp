@@ -20,8 +20,11 @@ extern const char* const rosenbrock_source;
 
 namespace {
 constexpr int kPollEvery = 8;
-// Reactors of a large mechanism up to which the batch is one part (53 species, us a step, one part against four: 100
-// reactors 591 against 695, 1000 661 against 726, 4000 934 against 922, 16000 2197 against 2161).
+// Reactors of a large mechanism up to which the batch is one part. us a step, one part against four on hardware queues of
+// their own: 53 species, 100 reactors 591 against 695, 1000 661 against 726, 4000 934 against 922, 16000 2197 against 2161;
+// 33 species 329 against 334 at 200 and 351 against 373 at 2048, 40 391 against 408 and 455 against 487, 45 438 against 457
+// and 512 against 544, 60 608 against 639 and 767 against 783 (784 against 759 at 1500). Four parts take twice that where
+// other streams of the process share their queues.
 constexpr size_t kOnePart = 2048;
 // Waves of rosenbrock_steps up to which it is faster than the separate kernels: its programs use one lane in seven, so
 // that beyond four waves a SIMD the chip is busy with them (six species, us a step, whole against separate: 1000 reactors
@@ -404,8 +407,9 @@ long Integrator::advance(double* y, const double* P, double* t, double* h, int* 
         const size_t fields = count * 2 * m;
         device::check(hipModuleLaunchKernel(copies_kernel, (unsigned)((fields + 255) / 256), 1, 1, 256, 1, 1, 0, st, rargs, nullptr),
                       "launch rosenbrock_copies");
-        // in one part, the right-hand side at the raised temperature runs beside that of the copies
-        hipStream_t beside = parts_.size() == 1 ? sides_[0] : st;
+        // in one part of a large mechanism, the right-hand side at the raised temperature runs beside that of the copies (a
+        // batch of eight or fewer that fills one part of a small one is faster without: 101 against 105 us a step)
+        hipStream_t beside = parts_of(n) == 1 ? sides_[0] : st;
         if (beside != st) {
           device::check(hipEventRecord(fork_, st), "hipEventRecord");
           device::check(hipStreamWaitEvent(beside, fork_, 0), "hipStreamWaitEvent");
