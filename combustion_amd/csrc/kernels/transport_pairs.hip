@@ -20,7 +20,7 @@
 // (the waves wait for their constants 60 % of theirs): 2^17 states take 0.99 ms against 2.09 ms for transport_tiled, whose
 // FP64 MFMA tiles have the VALU's rate on this chip and do not overlap it. Measured and not kept: half a column's
 // constants fetched ahead of the other half's arithmetic (1.04 ms: 106 scalar registers do not hold both).
-// Required defines: K, R (rank), DD (fit length), WAVES (even).
+// Required defines: K, R (rank), DD (fit length), WAVES (a power of two).
 // Tables: rcp_W[K], W[K], fit_c[K][DD], fit_v[K][DD] (v scaled), columns[R][KC] = √(W_j/8) G_jr (KC = K rounded up to 8),
 // rows[WAVES][R][SW] = G_kr / √W_k, pairs[WAVES][..] = per wave its pairs' DD constants in the order of the phases
 // (c_1/c_0, .., 1/c_0; a slot without species: 0, .., 0), offset[WAVES] into it.
@@ -32,10 +32,16 @@ typedef const double __attribute__((address_space(4))) * table;  // read by scal
 #define KC ((K + 7) / 8 * 8)
 #define HALF (SW / 2)
 
-// 1/b: v_rcp_f64 (relative error below 2^-24) and one Newton step (2.2e-15)
+// 1/b: v_rcp_f64 (r, relative error e below 2^-24) times 1 + e + e² (error e³: the last rounding is all there is). A Newton
+// step, 1 + e, is always low, by 3e-16 on average, which the sums do not average out.
 __device__ __forceinline__ double rcp64(double b) {
-  const double r = __builtin_amdgcn_rcp(b);
-  return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+  const double r = __builtin_amdgcn_rcp(b), e = __builtin_fma(-b, r, 1.0);
+  return __builtin_fma(r, __builtin_fma(e, e, e), r);
+}
+// a/b, rounded once or nearly
+__device__ __forceinline__ double quotient(double a, double b) {
+  const double r = rcp64(b), q = a * r;
+  return __builtin_fma(__builtin_fma(-b, q, a), r, q);
 }
 // ln x for x > 0: x = 2^e m with m in [sqrt(1/2), sqrt(2)), log2 m = s P(s²) with s = (m-1)/(m+1) (the atanh series; P
 // the Chebyshev interpolant of degree 7, relative error 1.4e-17)
@@ -58,7 +64,7 @@ __device__ __forceinline__ double log64(double x) {
   p = __builtin_fma(p, z, 0x1.2776c50ee39dcp-1);
   p = __builtin_fma(p, z, 0x1.ec709dc3a047dp-1);
   p = __builtin_fma(p, z, 0x1.71547652b82fep+1);
-  return __builtin_fma(s, p, (double)e) * 0x1.62e42fefa39efp-1;
+  return __builtin_fma((double)e, 0x1.62e42fefa39efp-1, s * p * 0x1.62e42fefa39efp-1);
 }
 
 // 1/y of N values from one reciprocal of their product (prefix products, then back; the y are near 1)
@@ -101,12 +107,12 @@ __device__ __forceinline__ void column(table& t, const double* pw, double xj, do
 #pragma unroll
   for (int i = 0; i < N * DD; i++) c[i] = t[i];
   t += N * DD;
-  double s = *sj;
+  double s = 0.0;  // the column's own sum first: a chain of all the pairs of j would round at the size of S_j each time
   reciprocals<A>(c, pw, ra);
 #pragma unroll
   for (int i = 0; i < A; i++) {
     g[i] = __builtin_fma(xj, ra[i], g[i]);
-    s = __builtin_fma(x[i], ra[i], s);
+    s = i ? __builtin_fma(x[i], ra[i], s) : x[i] * ra[i];
   }
   if constexpr (B > 0) {
     double rb[B];
@@ -117,14 +123,27 @@ __device__ __forceinline__ void column(table& t, const double* pw, double xj, do
       s = __builtin_fma(x[A + i], rb[i], s);
     }
   }
-  *sj = s;
+  *sj += s;
+}
+
+// The waves' values in the rows p[64 w], added in pairs
+__device__ __forceinline__ double waves_sum(const double* p) {
+  double v[WAVES];
+#pragma unroll
+  for (int w = 0; w < WAVES; w++) v[w] = p[64 * w];
+#pragma unroll
+  for (int n = WAVES / 2; n > 0; n /= 2) {
+#pragma unroll
+    for (int w = 0; w < n; w++) v[w] += v[w + n];
+  }
+  return v[0];
 }
 
 extern "C" __global__ void __launch_bounds__(64 * WAVES)
 transport_tiled(const double* const* __restrict__ in, double* const* __restrict__ out, unsigned n, const double* __restrict__ rcp_W_,
                 const double* __restrict__ W_, const double* __restrict__ fit_c_, const double* __restrict__ fit_v_,
                 const double* __restrict__ columns_, const double* __restrict__ rows_, const double* __restrict__ pairs_,
-                const unsigned* __restrict__ offset, double rcp_T0) {
+                const unsigned* __restrict__ offset, double T0) {
   __shared__ double lds_x[(K - 1) * 64];  // x_k without the bulk species'
   __shared__ double lds_s[K * 64];        // 1/v_k, then Gᵀ y_m, then S_k
   const table rcp_W = (table)rcp_W_, W = (table)W_, fit_c = (table)fit_c_, fit_v = (table)fit_v_;
@@ -154,22 +173,16 @@ transport_tiled(const double* const* __restrict__ in, double* const* __restrict_
   s_[wave * 64] = sum;
   s_[(WAVES + wave) * 64] = positive;
   s_[(2 * WAVES + wave) * 64] = mass;
-  const double l = log64(T * rcp_T0), C_tot = P * (1.0 / RGAS) * rcp64(T);
+  const double l = log64(T / T0), C_tot = quotient(quotient(P, RGAS), T);
   double pw[DD];
   pw[0] = 1.0;
 #pragma unroll
   for (int d = 1; d < DD; d++) pw[d] = pw[d - 1] * l;
   __syncthreads();
-  sum = s_[0];
-  positive = s_[WAVES * 64];
-  mass = s_[2 * WAVES * 64];
-#pragma unroll
-  for (int w = 1; w < WAVES; w++) {
-    sum += s_[w * 64];
-    positive += s_[(WAVES + w) * 64];
-    mass += s_[(2 * WAVES + w) * 64];
-  }
-  const double density = C_tot * rcp64(sum), bulk = C_tot - density * positive;
+  sum = waves_sum(s_);
+  positive = waves_sum(s_ + WAVES * 64);
+  mass = waves_sum(s_ + 2 * WAVES * 64);
+  const double density = quotient(C_tot, sum), bulk = C_tot - density * positive;
   const double WN = density * mass + W[K - 1] * bulk;  // Σ W_k x_k
   __syncthreads();
   double v[SW], A = 0.0, B = 0.0;
@@ -186,7 +199,7 @@ transport_tiled(const double* const* __restrict__ in, double* const* __restrict_
         u += fit_v[k * DD + d] * pw[d];
       }
       A += x[i] * c;
-      B += x[i] * rcp64(c);
+      B += quotient(x[i], c);
       v[i] = u;
       if (k < K - 1) lds_x[k * 64 + lane] = x[i];
       s_[k * 64] = rcp64(u);
@@ -205,15 +218,18 @@ transport_tiled(const double* const* __restrict__ in, double* const* __restrict_
       const table c = (table)columns_ + r * KC;
 #pragma unroll 1
       for (int j0 = 0; j0 < K; j0 += 8) {
+        double part[3];  // eight species first, for the same reason as a column's sum
 #pragma unroll
         for (int j = 0; j < 8; j++) {
           // past the species: a constant of zero, and the bulk's concentration
           const int k = j0 + j < K ? j0 + j : K - 1;
           const double xj = k < K - 1 ? x_[k * 64] : bulk, u = s_[k * 64], y1 = xj * u;
-          z[q][0] = __builtin_fma(c[j0 + j], xj, z[q][0]);
-          z[q][1] = __builtin_fma(c[j0 + j], y1, z[q][1]);
-          z[q][2] = __builtin_fma(c[j0 + j], y1 * u, z[q][2]);
+          part[0] = j ? __builtin_fma(c[j0 + j], xj, part[0]) : c[j0] * xj;
+          part[1] = j ? __builtin_fma(c[j0 + j], y1, part[1]) : c[j0] * y1;
+          part[2] = j ? __builtin_fma(c[j0 + j], y1 * u, part[2]) : c[j0] * (y1 * u);
         }
+#pragma unroll
+        for (int m = 0; m < 3; m++) z[q][m] += part[m];
       }
     }
   }
@@ -252,7 +268,7 @@ transport_tiled(const double* const* __restrict__ in, double* const* __restrict_
     }
 #pragma unroll
     for (int i = 0; i < SW; i++)
-      if (wave + WAVES * i < K) mu += x[i] * (v[i] * v[i]) * rcp64(d0[i] + v[i] * (2.0 * d1[i] + v[i] * d2[i]));
+      if (wave + WAVES * i < K) mu += quotient(x[i] * (v[i] * v[i]), d0[i] + v[i] * (2.0 * d1[i] + v[i] * d2[i]));
   }
   __syncthreads();
 #pragma unroll
@@ -312,23 +328,17 @@ transport_tiled(const double* const* __restrict__ in, double* const* __restrict_
   if (s >= n) return;
   const double root_T = __builtin_sqrt(T);
   if (wave == 0) {
-#pragma unroll
-    for (int w = 1; w < WAVES; w++) {
-      A += p_[w * 64];
-      B += p_[(WAVES + w) * 64];
-    }
-    out[0][s] = 0.5 * root_T * (A * rcp64(C_tot) + C_tot * rcp64(B));
+    A = waves_sum(p_);
+    B = waves_sum(p_ + WAVES * 64);
+    out[0][s] = 0.5 * root_T * (quotient(A, C_tot) + quotient(C_tot, B));
   }
   if (wave == 1) {
-    mu = p_[2 * WAVES * 64];
-#pragma unroll
-    for (int w = 1; w < WAVES; w++) mu += p_[(2 * WAVES + w) * 64];
-    out[1][s] = root_T * mu;
+    out[1][s] = root_T * waves_sum(p_ + 2 * WAVES * 64);
   }
-  const double scale = root_T * rcp64(RGAS * WN);
+  const double scale = quotient(root_T, RGAS * WN);
 #pragma unroll
   for (int i = 0; i < SW; i++) {
     const int k = wave + WAVES * i;
-    if (k < K) out[2 + k][s] = scale * (WN - W[k] * x[i]) * rcp64(g[i]);
+    if (k < K) out[2 + k][s] = quotient(scale * (WN - W[k] * x[i]), g[i]);
   }
 }

@@ -853,7 +853,7 @@ class RatesAndTransport {
 // transport_pairs with its tables in device memory; writes [λ, μ, D_0..D_{K-1}] to out[0..K+2).
 class TransportPairsKernel {
  public:
-  TransportPairsKernel(TransportPairs t, double T0) : t_(std::move(t)), rcp_T0_(1. / T0) {
+  TransportPairsKernel(TransportPairs t, double T0) : t_(std::move(t)), T0_(T0) {
     kernel_.load(device::compile(t_.source, "transport_tiled", hip_options(true)), "transport_tiled");
     for (const auto* v : {&t_.rcp_W, &t_.W, &t_.fit_c, &t_.fit_v, &t_.columns, &t_.rows, &t_.pairs}) tables_.push_back(upload(*v));
     d_offset_ = upload(t_.offset);
@@ -864,14 +864,14 @@ class TransportPairsKernel {
   }
   void launch(const double* const* in, double* const* out, size_t n, hipStream_t stream) {
     unsigned n32 = (unsigned)n;
-    void* args[] = {&in, &out, &n32, &tables_[0], &tables_[1], &tables_[2], &tables_[3], &tables_[4], &tables_[5], &tables_[6], &d_offset_, &rcp_T0_};
+    void* args[] = {&in, &out, &n32, &tables_[0], &tables_[1], &tables_[2], &tables_[3], &tables_[4], &tables_[5], &tables_[6], &d_offset_, &T0_};
     device::check(hipModuleLaunchKernel(kernel_.function, (unsigned)((n + 63) / 64), 1, 1, 64 * t_.waves, 1, 1, 0, stream, args, nullptr),
                   "launch transport");
   }
 
  private:
   TransportPairs t_;
-  double rcp_T0_;
+  double T0_;
   device::Kernel kernel_;
   std::vector<double*> tables_;
   unsigned* d_offset_ = nullptr;

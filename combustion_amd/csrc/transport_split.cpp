@@ -130,7 +130,7 @@ class Pairs {
 
 }  // namespace
 
-std::vector<double> wilke_factor(const std::vector<double>& W) {
+std::vector<long double> wilke_factor(const std::vector<double>& W) {
   const size_t K = W.size();
   auto entry = [&](size_t k, size_t j) { return 1.L / std::sqrt((long double)W[k] + (long double)W[j]); };
   std::vector<long double> rest(K);
@@ -152,9 +152,9 @@ std::vector<double> wilke_factor(const std::vector<double>& W) {
     columns.push_back(c);
   }
   const size_t R = columns.size();
-  std::vector<double> G(K * R);
+  std::vector<long double> G(K * R);
   for (size_t k = 0; k < K; k++)
-    for (size_t r = 0; r < R; r++) G[k * R + r] = (double)columns[r][k];
+    for (size_t r = 0; r < R; r++) G[k * R + r] = columns[r][k];
   return G;
 }
 
@@ -162,7 +162,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
   TransportSplit t;
   const std::vector<double>& W = m.species.molar_mass;
   const size_t K = W.size(), D = p.D;
-  const std::vector<double> G = wilke_factor(W);
+  const std::vector<long double> G = wilke_factor(W);
   const size_t R = G.size() / K, KW = (K + kWaves - 1) / kWaves;
   auto slots = [&](int wave) {
     std::vector<int> v;
@@ -184,7 +184,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
         read << "  const double x" << j << " = X(" << j << "), u" << j << " = S(" << j << ");\n";
         text << "  { const double y1 = x" << j << " * u" << j << ", y2 = y1 * u" << j << ";\n";
         for (size_t i = 0; kWaves * i + w < R; i++) {
-          const std::string c = literal(G[j * R + kWaves * i + w] * std::sqrt(W[j] / 8.));
+          const std::string c = literal((double)(G[j * R + kWaves * i + w] * std::sqrt(W[j] / 8.L)));
           for (int mth = 0; mth < 3; mth++)
             text << term("z[" + std::to_string(i) + "][" + std::to_string(mth) + "]", c, mth == 0 ? "x" + std::to_string(j) : "y" + std::to_string(mth), j == 0);
         }
@@ -200,7 +200,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
       for (int mth = 0; mth < 3; mth++) read << "  const double z" << q << "_" << mth << " = S(" << 3 * q + mth << ");\n";
       for (int i : slots(w)) {
         const size_t k = kWaves * i + w;
-        const std::string c = literal(G[k * R + q] / std::sqrt(W[k]));
+        const std::string c = literal((double)(G[k * R + q] / std::sqrt((long double)W[k])));
         for (int mth = 0; mth < 3; mth++) text << term("d" + std::to_string(mth) + "[" + std::to_string(i) + "]", c, "z" + std::to_string(q) + "_" + std::to_string(mth), q == 0);
       }
       r.add(read.str(), text.str());
@@ -236,7 +236,7 @@ TransportSplit transport_split(const Mechanism& m, const Polynomials& p) {
     t.W.push_back(W[k]);
     for (size_t d = 0; d < D; d++) {
       t.fit_c.push_back(p.conductivityIVT[k * D + d]);
-      t.fit_v.push_back(p.VviscosityIVVT[k * D + d] / std::sqrt(std::sqrt(W[k])));
+      t.fit_v.push_back((double)(p.VviscosityIVVT[k * D + d] / std::sqrt(std::sqrt((long double)W[k]))));
     }
   }
   return t;
@@ -246,7 +246,7 @@ TransportPairs transport_pairs(const Mechanism& m, const Polynomials& p) {
   TransportPairs t;
   const std::vector<double>& W = m.species.molar_mass;
   const size_t K = W.size(), D = p.D, waves = t.waves, slots = (K + waves - 1) / waves, half = slots / 2;
-  const std::vector<double> G = wilke_factor(W);
+  const std::vector<long double> G = wilke_factor(W);
   const size_t R = G.size() / K, KC = (K + 7) / 8 * 8;
   // the two LDS arrays, the rows of the waves' partial sums in them, and fits that can be normalised
   bool fits = slots >= 4 && (2 * K - 1) * 64 * sizeof(double) <= 160 * 1024 && K > 3 * waves && 3 * R <= K && D >= 2;
@@ -261,16 +261,16 @@ TransportPairs transport_pairs(const Mechanism& m, const Polynomials& p) {
     t.W.push_back(W[k]);
     for (size_t d = 0; d < D; d++) {
       t.fit_c.push_back(p.conductivityIVT[k * D + d]);
-      t.fit_v.push_back(p.VviscosityIVVT[k * D + d] / std::sqrt(std::sqrt(W[k])));
+      t.fit_v.push_back((double)(p.VviscosityIVVT[k * D + d] / std::sqrt(std::sqrt((long double)W[k]))));
     }
   }
   t.columns.assign(R * KC, 0.);
   for (size_t r = 0; r < R; r++)
-    for (size_t j = 0; j < K; j++) t.columns[r * KC + j] = G[j * R + r] * std::sqrt(W[j] / 8.);
+    for (size_t j = 0; j < K; j++) t.columns[r * KC + j] = (double)(G[j * R + r] * std::sqrt(W[j] / 8.L));
   t.rows.assign(waves * R * slots, 0.);
   for (size_t w = 0; w < waves; w++)
     for (size_t r = 0; r < R; r++)
-      for (size_t i = 0; w + waves * i < K; i++) t.rows[(w * R + r) * slots + i] = G[(w + waves * i) * R + r] / std::sqrt(W[w + waves * i]);
+      for (size_t i = 0; w + waves * i < K; i++) t.rows[(w * R + r) * slots + i] = (double)(G[(w + waves * i) * R + r] / std::sqrt((long double)W[w + waves * i]));
   // pairs of the wave's slot i (species k) with species j, a slot without species giving no term
   auto pair = [&](size_t k, size_t j) {
     const double* c = k < K && j < K ? &p.diffusivityITVT[(k * K + j) * D] : nullptr;

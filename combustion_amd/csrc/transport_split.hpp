@@ -24,6 +24,6 @@ struct TransportPairs {
 TransportPairs transport_pairs(const Mechanism& m, const Polynomials& p);
 
 // Factor G [K][R] with G Gᵀ = 1/√(W_k + W_j) to 2^-56 of every entry (pivoted Cholesky, row-major; R is its size / K).
-std::vector<double> wilke_factor(const std::vector<double>& W);
+std::vector<long double> wilke_factor(const std::vector<double>& W);
 
 }  // namespace combustion
