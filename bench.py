@@ -395,7 +395,7 @@ def main():
         fp64(host_in, host_out)
     host_s = (time.perf_counter() - t0) / 3
     result["pcie_inclusive"] = {"states_per_s": N / host_s, "ms_per_step": host_s * 1e3,
-                                "note": "host numpy buffers through cb_hip_call (pageable memory, blocking); not the value"}
+                                "note": "host numpy buffers through cb_hip_call (pageable arrays through the module's pinned slices, blocking); not the value"}
 
     # the nekRK export (cuda.rs:296-337): the four emitted files compiled by hiprtc and run as one kernel over the same
     # states (fits of length 5, the reference's export length), timed like the forms

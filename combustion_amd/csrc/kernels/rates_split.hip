@@ -12,16 +12,16 @@
 //   3. the parts' sums, in a fixed order: the upper half of the parts hands its sums to the lower half through LDS,
 //      then every part adds the rows of its own species and writes them out
 //
-// Bound: FP64 VALU issue. Per 64 states of the 53-species mechanism it issues 17.3 k VALU instructions where the
+// Bound: FP64 VALU issue. Per 64 states of the 53-species mechanism it issues 17.5 k VALU instructions where the
 // one-lane kernel issued 23.4 k (no accumulation-register moves, exponentials without clamps of their own and with
-// a reduction of one rounding, one exponential per rate constant, one factor per product species) at one wave per SIMD; with two waves per SIMD and the
-// parts' scalar constants and LDS reads beside the other wave's arithmetic, 2^20 states take 0.80 ms against 1.19 ms,
-// and a single wavefront's worth of states 25 against 75 us (a quarter of the reactions per wave). What is left of
-// it: a block of 128 states spends 34 of its 54 k cycles in the reactions (27 k of them issue), 7 k in the Gibbs
-// exponentials, 6 k on its loads and 4 k on the sums. Measured and not kept: six parts at three waves per SIMD (0.83
-// to 0.95 ms: 168 registers spill), persistent blocks with the teams on barriers of their own (0.82 to 0.9 ms: the
-// loop's invariants spill), rows of independent instructions pinned by scheduling barriers (0.80 ms, compile times of
-// minutes).
+// a reduction of one rounding, one exponential per rate constant, one factor per product species) at one wave per
+// SIMD; with two waves per SIMD and the parts' scalar constants and LDS reads beside the other wave's arithmetic, 2^20
+// states take 0.86 ms against 1.18 ms (30 launches each on one card; 0.92 in the full benchmark run), and a single
+// wavefront's worth of states 25 against 75 us (a quarter of the reactions per wave). What is left of it: two thirds of a
+// block's cycles are the reactions (half of them issue), an eighth the Gibbs exponentials, a tenth its loads and a
+// fourteenth the sums. Measured and not kept: six parts at three waves per SIMD (4 to 19 % longer: 168 registers spill),
+// persistent blocks with the teams on barriers of their own (2 to 12 % longer: the loop's invariants spill), rows of
+// independent instructions pinned by scheduling barriers (no gain, compile times of minutes).
 // Rounding: 3.6e-15 of the state's largest rate on average (4096 states, against the program in 80-bit arithmetic), 4.7e-15
 // for the one-lane kernel and 4.0e-15 with the library's functions.
 // Required defines: NAME, K, KA (active species), PARTS (waves per team, even), TEAMS (teams per block), FAST (1: exp

@@ -16,10 +16,14 @@
 // The pairs' constants are wave-uniform and used once: each wave streams its own through scalar loads, whose latency the
 // other three waves of its SIMD cover.
 //
-// Bound: FP64 VALU issue. 163 k VALU instructions per 64 states of 160 species, four waves per SIMD, VALU busy 67 % of the time
-// (the waves wait for their constants 60 % of theirs): 2^17 states take 0.99 ms against 2.09 ms for transport_tiled, whose
-// FP64 MFMA tiles have the VALU's rate on this chip and do not overlap it. Measured and not kept: half a column's
-// constants fetched ahead of the other half's arithmetic (1.04 ms: 106 scalar registers do not hold both).
+// Bound: FP64 VALU issue and the constants' latency. 171 k VALU instructions per 64 states of 160 species, four waves per
+// SIMD, VALU busy 63 % of the time (the waves wait 56 % of theirs, mostly for their constants): 2^17 states take 1.00 ms
+// against 2.09 ms for transport_tiled, whose FP64 MFMA tiles have the VALU's rate on this chip and do not overlap it.
+// Measured and not kept: half a column's constants fetched ahead of the other half's arithmetic (5 % longer: 106 scalar
+// registers do not hold both).
+// Rounding: 1.1e-16, 1.1e-16 and 1.9e-16 of λ, μ and ρD on average against the formulas in 80-bit arithmetic (160 species);
+// transport_tiled 1.3e-16, 1.4e-16 and 2.1e-16. The reciprocals, quotients and the order of the sums below are for that: they
+// took 4 % more instructions and 1.2 % of the time.
 // Required defines: K, R (rank), DD (fit length), WAVES (a power of two).
 // Tables: rcp_W[K], W[K], fit_c[K][DD], fit_v[K][DD] (v scaled), columns[R][KC] = √(W_j/8) G_jr (KC = K rounded up to 8),
 // rows[WAVES][R][SW] = G_kr / √W_k, pairs[WAVES][..] = per wave its pairs' DD constants in the order of the phases

@@ -15,10 +15,10 @@
 //       barriers). The fits normalised by their constant term, four reciprocals from one.
 // Bound: FP64 VALU issue (22.0 k VALU instructions per 64 states of the 53-species mechanism, 14.3 k of them for its 1378
 // pairs, where one lane per state took 26.2 k), at three waves per SIMD, which the 105 rows of LDS just allow (the bulk
-// species' x stays in a register for that). 2^20 states of 53 species: 0.96 ms against 1.04 ms for one lane per state
-// (VALU busy 77 % of the time); 64 states: 30 against 84 us. Measured and not kept: the sections' constants by scalar
-// loads one block ahead instead of s_mov pairs (1.31 ms: every wait for one is a wait for all), two waves per SIMD
-// (1.01 ms), FP64 MFMA for the moments (v_mfma_f64_16x16x4 has the VALU's rate on this chip and does not overlap it).
+// species' x stays in a register for that). 2^20 states of 53 species: 0.90 ms against 1.01 ms for one lane per state
+// (VALU busy 83 % of the time); 64 states: 30 against 84 us. Measured and not kept: the sections' constants by scalar
+// loads one block ahead instead of s_mov pairs (a third longer: every wait for one is a wait for all), two waves per
+// SIMD (11 % longer), FP64 MFMA for the moments (v_mfma_f64_16x16x4 has the VALU's rate on this chip and does not overlap it).
 // Required defines: K, R (rank), DD (fit length).
 // Tables: rcp_W[K], W[K], fit_c[K][DD], fit_v[K][DD] (v scaled).
 

@@ -21,8 +21,8 @@ constexpr double kLog2e = 1.4426950408889634;
 // A compiler-only fence between segments: each reads the LDS values it uses instead of keeping an earlier read live.
 const char* const kFence = "  asm volatile(\"\" ::: \"memory\");\n";
 // Reactions per segment. A segment's LDS values are read while the segment before it computes, and its reactions are
-// evaluated side by side, factor by factor. One and two reactions at a time took 0.84 and 0.81 ms per 2^20 states of
-// the 53-species mechanism, four 0.80 ms at 245 of the 256 registers.
+// evaluated side by side, factor by factor. One and two reactions at a time took 5 and 1 % longer than four (53 species),
+// which fill 251 of the 256 registers.
 constexpr size_t kSegment = 4, kThirdBodySegment = 2;
 
 std::string literal(double x) {
@@ -466,7 +466,7 @@ RatesSplit rates_split(const Mechanism& m, const std::string& name, bool fast, b
     if (!segments.empty()) s << segments[0].reads << kFence;
     for (size_t i = 0; i < segments.size(); i++) {
       // The older team's waves win the issue slots and would leave the younger one's to run alone at the end, one
-      // instruction per five cycles: the younger goes first for its first half (0.84 -> 0.80 ms).
+      // instruction per five cycles: the younger goes first for its first half (5 % of the kernel's time).
       if (i == 0 && t.teams > 1) s << "  if (team) __builtin_amdgcn_s_setprio(1);\n";
       if (i == segments.size() / 2 && t.teams > 1) s << "  __builtin_amdgcn_s_setprio(0);\n";
       s << (i + 1 < segments.size() ? segments[i + 1].reads + kFence : "") << segments[i].text;

@@ -542,8 +542,8 @@ RatesText rates_text(const ProgramView& p, bool fast) {
   RatesText t;
   t.name = fast ? "rates_fast" : "rates_fp64";
   const ast::Linear l = lean_rates(p);
-  // A program of more live doubles than the 128 that two waves per SIMD hold goes to teams of waves (53 species: 0.80
-  // against 1.19 ms per 2^20 states at one wave per SIMD); a smaller one runs without their LDS traffic and barriers.
+  // A program of more live doubles than the 128 that two waves per SIMD hold goes to teams of waves (53 species: 0.86
+  // against 1.18 ms per 2^20 states at one wave per SIMD); a smaller one runs without their LDS traffic and barriers.
   if (ast::peak_live(l) > 128) {
     t.split = rates_split(*p.mechanism, t.name, fast);
     t.source = t.split.source;
@@ -884,7 +884,10 @@ TransportPairs pairs_of(const ProgramView& p, int form_flags) {
   return transport_pairs(*p.mechanism, polynomials(p));
 }
 
-constexpr size_t kForkWork = size_t(1) << 27;  // states × species² from which two kernels of a call take two streams
+// states × species² from which two kernels of a call take two streams. The point was found at 53 species; below it one stream
+// was ahead of two at all of 64 to 2^20 states for 10 and 24 species in the fast and mixed forms (2^17 of 24: 69 against 120
+// us and 181 against 213).
+constexpr size_t kForkWork = size_t(1) << 27;
 
 class Tiled : public SoAForm {
  public:
